@@ -5,7 +5,7 @@
 // B operand wants 16 consecutive K bytes per lane, so the skinny core transposes weight bytes in
 // registers with v_perm_b32 (4x4 byte blocks) on their way from HBM.
 //
-//   skinny_kernel  decode-shaped groups (<= 16 rows per pass) of QuantMatmul and the int8 grouped
+//   skinny_kernel  decode-shaped groups (16 or 32 rows per pass over the weights) of QuantMatmul and the int8 grouped
 //                  down-projection (EPI_DEQUANT: the QuantMatmul dequant chain straight to bf16 /
 //                  fp16) and the int32 GEMM (EPI_I32).  One workgroup = (group, 256 weight
 //                  columns); its 4 waves split K, stream the weight block straight from HBM into
@@ -237,30 +237,36 @@ __device__ __forceinline__ SkinnyRow skinny_row(const GemmArgs& a, const int64_t
         s.res = make_rsrc(a.x + boff, (uint32_t)(a.x_rows * K));
         s.off = srow >= 0 ? (uint32_t)srow * (uint32_t)K : kSkOff;
     } else {
-        const int nrow = r1 - mb < 16 ? r1 - mb : 16;
+        const int nrow = r1 - mb < 16 ? (r1 - mb > 0 ? r1 - mb : 0) : 16;  // 0: a block past the group's end
         s.res = make_rsrc(a.x + boff + (int64_t)mb * K, (uint32_t)((int64_t)nrow * K));
         s.off = arow < r1 ? (uint32_t)c * (uint32_t)K : kSkOff;
     }
     return s;
 }
 
-// One 64-deep chunk of a skinny tile: the lane's activation operand (first, so waiting for it never
-// waits for weights issued later) and 16 weight rows; k past K (and rows outside the group) read as
-// zeros.
-__device__ __forceinline__ void skinny_load_chunk(const SkinnyRow& xr, __amdgpu_buffer_rsrc_t wres,
+// One 64-deep chunk of a skinny tile: the lane's activation operands of RB row blocks (first, so
+// waiting for them never waits for weights issued later) and 16 weight rows; k past K (and rows
+// outside the group) read as zeros.
+template <int RB>
+__device__ __forceinline__ void skinny_load_chunk(const SkinnyRow (&xr)[RB], __amdgpu_buffer_rsrc_t wres,
                                                   const uint32_t lane_off, const uint32_t n, const int q,
-                                                  const int kc, uint4 (&R)[16], v4i& A)
+                                                  const int kc, uint4 (&R)[16], v4i (&A)[RB])
 {
     const uint32_t k = (uint32_t)(kc * 64 + q * 16);
-    A = __builtin_amdgcn_raw_buffer_load_b128(xr.res, xr.off != kSkOff && k < xr.k ? xr.off + k : kSkOff, 0, 0);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+        A[rb] = __builtin_amdgcn_raw_buffer_load_b128(
+            xr[rb].res, xr[rb].off != kSkOff && k < xr[rb].k ? xr[rb].off + k : kSkOff, 0, 0);
     const uint32_t kofs = (uint32_t)(kc * 64) * n;
 #pragma unroll
     for (int i = 0; i < 16; ++i) R[i] = buf_load16(wres, lane_off + kofs + (uint32_t)i * n);
 }
 
 // The chunk's MFMAs: the 16 loaded rows are transposed in registers into 16 B operands, one per
-// column, and MFMA j accumulates column 16 c + j.
-__device__ __forceinline__ void skinny_mma_chunk(const uint4 (&R)[16], const v4i av, v4i (&acc)[16])
+// column, and MFMA j of row block rb accumulates column 16 c + j; the weights are transposed once
+// for all row blocks.
+template <int RB>
+__device__ __forceinline__ void skinny_mma_chunk(const uint4 (&R)[16], const v4i (&av)[RB], v4i (&acc)[RB][16])
 {
     // column block cb: the 4 B operands of columns 4 cb .. 4 cb + 3, built from dword cb of the 16
     // loaded rows, consumed right away to keep the live range short
@@ -279,8 +285,37 @@ __device__ __forceinline__ void skinny_mma_chunk(const uint4 (&R)[16], const v4i
         }
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4)
-            acc[4 * cb + s4] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, as_v4i(T[s4]), acc[4 * cb + s4], 0, 0, 0);
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+                acc[rb][4 * cb + s4] =
+                    __builtin_amdgcn_mfma_i32_16x16x64_i8(av[rb], as_v4i(T[s4]), acc[rb][4 * cb + s4], 0, 0, 0);
     }
+}
+
+// Exact K reduction of one row block over the 4 waves that split K: wave w keeps accumulator row w
+// (s[j] = C[row 4 q + w][column 16 c + j]) and receives the other waves' partials through red.
+// Ends with a barrier: red may be reused.
+__device__ __forceinline__ void skinny_reduce(const v4i (&acc)[16], int (&red)[3][4][16][64], const int wave,
+                                              const int lane, int (&s)[16])
+{
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (r != wave) {
+            const int slot = wave < r ? wave : wave - 1;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) red[slot][r][j][lane] = acc[j][r];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        int v = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (r == wave) v = acc[j][r];
+        s[j] = v + red[0][wave][j][lane] + red[1][wave][j][lane] + red[2][wave][j][lane];
+    }
+    __syncthreads();
 }
 
 // Epilogue of one output row of a skinny tile: lane (q, c) holds s[j] = C[row][ocol + j] (SwiGLU:
@@ -317,6 +352,18 @@ __device__ __forceinline__ void skinny_row_epilogue(const GemmArgs& a, const int
     }
 }
 
+// Group of row tile mt in a GroupTable enumeration.
+__device__ __forceinline__ int group_of_tile(const GroupTable& gt, int mt)
+{
+    int lo = 0, hi = gt.n_groups - 1;
+    while (lo < hi) {  // last g with tile_start[g] <= mt and a non-empty tile range
+        const int mid = (lo + hi + 1) >> 1;
+        if (gt.tile_start[mid] <= mt) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
 // Block -> (group, column tile) of the skinny kernels.  a.xcd_split = P > 0: XCD pair / quad p
 // streams groups p, p + 8 / P, ... and each of its P XCDs one contiguous 1 / P of their column
 // tiles (workgroups are dispatched round-robin over the 8 XCDs in linear block order).
@@ -341,7 +388,7 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& a, int& g, int& ct)
 //   group c = l % 16 (16 consecutive weight columns); after the in-register 16x16 byte transpose
 //   the lane holds 16 B operands, one per column, and MFMA j yields column (16 c + j).
 // ============================================================================================
-template <int EPI>
+template <int EPI, int RB>
 __global__ __launch_bounds__(256, 2) void skinny_kernel(const GemmArgs a)
 {
     __shared__ int red[3][4][16][64];  // partial sums handed to the wave that owns them (48 KiB)
@@ -371,67 +418,34 @@ __global__ __launch_bounds__(256, 2) void skinny_kernel(const GemmArgs a)
     const uint32_t lane_off = (uint32_t)(colok ? col : 0) + (uint32_t)(q * 16) * (uint32_t)N;
     const int nch = (int)((K + 63) >> 6);
 
-    for (int mb = r0; mb < r1; mb += 16) {
-        v4i acc[16];
+    for (int mb = r0; mb < r1; mb += 16 * RB) {
+        v4i acc[RB][16];
+        // activation row of this lane in each row block: rows past the group (or gathered from
+        // outside x) and k past K read as zeros without a branch, so the activation loads join
+        // their chunk's weight loads
+        SkinnyRow xres[RB];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) acc[j] = v4i{0, 0, 0, 0};
-
-        // activation row of this lane: rows past the group (or gathered from outside x) and k past
-        // K read as zeros without a branch, so the activation load joins its chunk's weight loads
-        const SkinnyRow xres = skinny_row(a, b * a.x_bstride, mb, r1, c);
-
-        // one chunk = the activation operand (first, so waiting for it never waits for weights
-        // issued later) and 16 weight rows
-        auto load_chunk = [&](int kc, uint4 (&R)[16], v4i& A) {
-            skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, kc, R, A);
-        };
-        auto mma_chunk = [&](const uint4 (&R)[16], const v4i av) { skinny_mma_chunk(R, av, acc); };
-
+        for (int rb = 0; rb < RB; ++rb) {
+            xres[rb] = skinny_row(a, b * a.x_bstride, mb + 16 * rb, r1, c);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) acc[rb][j] = v4i{0, 0, 0, 0};
+        }
         for (int kc = wave; kc < nch; kc += 4) {
             uint4 R[16];
-            v4i A;
-            load_chunk(kc, R, A);
-            mma_chunk(R, A);
+            v4i A[RB];
+            skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, kc, R, A);
+            skinny_mma_chunk(R, A, acc);
         }
-
-        // Cross-wave K reduction: wave w keeps accumulator row r == w and receives the other
-        // three waves' partials for it through LDS.
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (r != wave) {
-                const int slot = wave < r ? wave : wave - 1;
-#pragma unroll
-                for (int j = 0; j < 16; ++j) red[slot][r][j][lane] = acc[j][r];
-            }
+        for (int rb = 0; rb < RB; ++rb) {
+            if (rb && mb + 16 * rb >= r1) break;  // uniform
+            int s[16];
+            skinny_reduce(acc[rb], red, wave, lane, s);
+            // MFMA 16x16 C layout: lane l holds rows 4 (l / 16) + r, column l % 16.
+            const int row = mb + 16 * rb + 4 * q + wave;
+            skinny_row_epilogue<EPI>(a, g, b, row, row < r1, colok, ocol, col, c, s);
         }
-        __syncthreads();
-        int s[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            int v = 0;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (r == wave) v = acc[j][r];
-            s[j] = v + red[0][wave][j][lane] + red[1][wave][j][lane] + red[2][wave][j][lane];
-        }
-        __syncthreads();  // the next row block reuses red[]
-
-        // MFMA 16x16 C layout: lane l holds rows 4 (l / 16) + r, column l % 16.
-        const int row = mb + 4 * q + wave;
-        skinny_row_epilogue<EPI>(a, g, b, row, row < r1, colok, ocol, col, c, s);
     }
-}
-
-// Group of row tile mt in a GroupTable enumeration.
-__device__ __forceinline__ int group_of_tile(const GroupTable& gt, int mt)
-{
-    int lo = 0, hi = gt.n_groups - 1;
-    while (lo < hi) {  // last g with tile_start[g] <= mt and a non-empty tile range
-        const int mid = (lo + hi + 1) >> 1;
-        if (gt.tile_start[mid] <= mt) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
 }
 
 // ============================================================================================

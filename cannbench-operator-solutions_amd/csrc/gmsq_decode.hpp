@@ -18,12 +18,18 @@
 
 namespace cb {
 
-// The product, SwiGLU and row maxima of one (expert g, 128-act-column) tile.  Lane (q, c), c < 8,
-// ends with act[rb][j] = act of row r0 + 16 rb + 4 q + wave, act column 128 ct + 16 c + j, and
-// rmax[rb] = the row's maximum |act| over the tile (in every lane of the 16-lane group); lanes
-// c >= 8 hold the up partners during the product and zeros after.
-__device__ __forceinline__ void decode_tile_act(const GemmArgs& a, const int g, const int ct, const int r0, const int r1,
-                                                int (&red)[3][4][16][64], float (&act)[2][16], u32 (&rmax)[2])
+// The product, SwiGLU and row maxima of one tile: RB 16-row blocks of expert g from row r0 on (rows
+// below r1) x 128 act columns.  Lane (q, c), c < 8, ends with act[rb][j] = act of row r0 + 16 rb +
+// 4 q + wave, act column 128 ct + 16 c + j, and rmax[rb] = the row's maximum |act| over the tile (in
+// every lane of the 16-lane group); lanes c >= 8 hold the up partners during the product and zeros
+// after.  The weights are streamed and transposed once for all RB row blocks: the kernel is bound by
+// the weight stream, and a second pass for rows 17 to 32 doubled it (7168 x 4096 x 256 experts with
+// 16 rows each on average, 28 at most: 1.55 ms, 1.18 ms in one pass; 2048 rows, 16 at most: 1.16 ms
+// either way).
+template <int RB, int RBM>
+__device__ __forceinline__ void decode_tile_act_n(const GemmArgs& a, const int g, const int ct, const int r0,
+                                                  const int r1, int (&red)[3][4][16][64], float (&act)[RBM][16],
+                                                  u32 (&rmax)[RBM])
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int q = lane >> 4, c = lane & 15;
@@ -37,52 +43,40 @@ __device__ __forceinline__ void decode_tile_act(const GemmArgs& a, const int g, 
     const __amdgpu_buffer_rsrc_t wres = make_rsrc(a.w + (int64_t)g * a.w_gstride, (uint32_t)(K * N));
     const uint32_t lane_off = (uint32_t)(colok ? col : 0) + (uint32_t)(q * 16) * (uint32_t)N;
     const int nch = (int)((K + 63) >> 6);
+    v4i acc[RB][16];
+    SkinnyRow xres[RB];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; rb < RB; ++rb) {
+        xres[rb] = skinny_row(a, 0, r0 + 16 * rb, r1, c);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[rb][j] = v4i{0, 0, 0, 0};
+    }
+    // wave w multiplies chunks w, w + 4, ...; two chunks in flight per wave (register double
+    // buffering): the load of chunk kc + 8 goes out as soon as chunk kc is multiplied.  Chunks
+    // past K read zeros through both resources (their MFMAs add nothing), so the loop needs no
+    // branch around a load.
+    uint4 R0[16], R1[16];
+    v4i A0[RB], A1[RB];
+    skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, wave, R0, A0);
+    skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, wave + 4, R1, A1);
+    for (int kc = wave; kc < nch; kc += 8) {
+        skinny_mma_chunk(R0, A0, acc);
+        skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, kc + 8, R0, A0);
+        skinny_mma_chunk(R1, A1, acc);
+        skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, kc + 12, R1, A1);
+    }
+#pragma unroll
+    for (int rb = 0; rb < RBM; ++rb) {
         rmax[rb] = 0u;
 #pragma unroll
         for (int j = 0; j < 16; ++j) act[rb][j] = 0.0f;
-        const int mb = r0 + 16 * rb;
-        if (mb >= r1) continue;  // uniform
-        v4i acc[16];
+    }
 #pragma unroll
-        for (int j = 0; j < 16; ++j) acc[j] = v4i{0, 0, 0, 0};
-        const SkinnyRow xres = skinny_row(a, 0, mb, r1, c);
-        // wave w multiplies chunks w, w + 4, ...; two chunks in flight per wave (register double
-        // buffering): the load of chunk kc + 8 goes out as soon as chunk kc is multiplied.  Chunks
-        // past K read zeros through both resources (their MFMAs add nothing), so the loop needs no
-        // branch around a load.
-        uint4 R0[16], R1[16];
-        v4i A0, A1;
-        skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, wave, R0, A0);
-        skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, wave + 4, R1, A1);
-        for (int kc = wave; kc < nch; kc += 8) {
-            skinny_mma_chunk(R0, A0, acc);
-            skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, kc + 8, R0, A0);
-            skinny_mma_chunk(R1, A1, acc);
-            skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, kc + 12, R1, A1);
-        }
-        // exact cross-wave K reduction: wave w keeps accumulator row w
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (r != wave) {
-                const int slot = wave < r ? wave : wave - 1;
-#pragma unroll
-                for (int j = 0; j < 16; ++j) red[slot][r][j][lane] = acc[j][r];
-            }
-        }
-        __syncthreads();
+    for (int rb = 0; rb < RB; ++rb) {
+        if (r0 + 16 * rb >= r1) continue;  // uniform
         int s[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            int v = 0;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (r == wave) v = acc[j][r];
-            s[j] = v + red[0][wave][j][lane] + red[1][wave][j][lane] + red[2][wave][j][lane];
-        }
-        __syncthreads();  // the next row block reuses red[]
-        const int row = mb + 4 * q + wave;
+        skinny_reduce(acc[rb], red, wave, lane, s);
+        const int row = r0 + 16 * rb + 4 * q + wave;
         int u[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) u[j] = __shfl_xor(s[j], 8, 64);
@@ -104,17 +98,28 @@ __device__ __forceinline__ void decode_tile_act(const GemmArgs& a, const int g, 
     }
 }
 
+// The smallest variant that holds the tile's rows.
+template <int RBM>
+__device__ __forceinline__ void decode_tile_act(const GemmArgs& a, const int g, const int ct, const int r0, const int r1,
+                                                int (&red)[3][4][16][64], float (&act)[RBM][16], u32 (&rmax)[RBM])
+{
+    if (r1 - r0 <= 16) decode_tile_act_n<1>(a, g, ct, r0, r1, red, act, rmax);
+    else if (RBM == 2 || r1 - r0 <= 32) decode_tile_act_n<2>(a, g, ct, r0, r1, red, act, rmax);
+    else if constexpr (RBM > 2) decode_tile_act_n<RBM>(a, g, ct, r0, r1, red, act, rmax);
+}
+
 // Row maxima exchange through self-validating slots: tile (g, ct) stores, for each of its rows r,
 // slot[r * ntiles + ct] = |act| maximum bits | 0x80000000 (the bit marks the slot as written; the
 // workspace starts zeroed).  A row's final maximum is the maximum over its ntiles slots once every
 // slot carries the mark, so no separate arrival count (and no wait for the stores) is needed.
+template <int RBM>
 __device__ __forceinline__ void decode_publish(const GemmArgs& a, const int ct, const int r0, const int r1,
-                                               const u32 (&rmax)[2])
+                                               const u32 (&rmax)[RBM])
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int q = lane >> 4, c = lane & 15;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; rb < RBM; ++rb) {
         const int row = r0 + 16 * rb + 4 * q + wave;
         if (c == 0 && row < r1)
             __hip_atomic_store(a.epi.amax + (int64_t)row * a.ntiles + ct, rmax[rb] | 0x80000000u, __ATOMIC_RELAXED,
@@ -124,7 +129,8 @@ __device__ __forceinline__ void decode_publish(const GemmArgs& a, const int ct, 
 
 // The final row maxima of this lane's rows (every lane of a 16-lane group gets its row's value),
 // polling until all ntiles slots are marked, at most spin_limit times.  Returns false on timeout.
-__device__ __forceinline__ bool decode_gather(const GemmArgs& a, const int r0, const int r1, float (&am)[2])
+template <int RBM>
+__device__ __forceinline__ bool decode_gather(const GemmArgs& a, const int r0, const int r1, float (&am)[RBM])
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int q = lane >> 4, c = lane & 15;
@@ -132,7 +138,7 @@ __device__ __forceinline__ bool decode_gather(const GemmArgs& a, const int r0, c
     for (int spins = 0;; ++spins) {
         bool all = true;
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
+        for (int rb = 0; rb < RBM; ++rb) {
             const int row = r0 + 16 * rb + 4 * q + wave;
             u32 m = 0u, ok = 1u;
             if (r0 + 16 * rb < r1 && row < r1) {
@@ -165,8 +171,9 @@ __device__ __forceinline__ bool decode_gather(const GemmArgs& a, const int r0, c
 
 // y = rint16(act * 127 / amax) with amax floored at FLT_MIN (an all-zero row gives 0 * inf = NaN
 // -> 0), 16 bytes per lane; column tile 0 writes y_scale.
+template <int RBM>
 __device__ __forceinline__ void decode_tile_quant(const GemmArgs& a, const int ct, const int r0, const int r1,
-                                                  const float (&act)[2][16], const float (&amax)[2])
+                                                  const float (&act)[RBM][16], const float (&amax)[RBM])
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int q = lane >> 4, c = lane & 15;
@@ -174,7 +181,7 @@ __device__ __forceinline__ void decode_tile_quant(const GemmArgs& a, const int c
     const int64_t H = e.H;
     const int64_t ocol = (int64_t)ct * 128 + 16 * (c & 7);
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; rb < RBM; ++rb) {
         const int row = r0 + 16 * rb + 4 * q + wave;
         if (row < r1) {
             float am = amax[rb];
@@ -208,16 +215,17 @@ __device__ __forceinline__ void decode_tile_quant(const GemmArgs& a, const int c
 // for the fix-up launch (which redoes the whole tile) and stores nothing.  no_wait: the tile is
 // left to the fix-up launch without waiting (status bit 1 instead of the timeout bit 0, so the
 // other waits of the call still wait).
-__device__ __forceinline__ void decode_finish(const GemmArgs& a, const int g, const int ct, const int r0, const int r1,
-                                              const float (&act)[2][16], const bool no_wait = false)
+template <int RBM>
+__device__ __forceinline__ void decode_finish(const GemmArgs& a, const int mt, const int ct, const int r0, const int r1,
+                                              const float (&act)[RBM][16], const bool no_wait = false)
 {
-    float am[2];
+    float am[RBM];
     // a negative poll limit (test hook) gives up at once
     if (!no_wait && a.epi.spin_limit >= 0 && decode_gather(a, r0, r1, am)) {
         decode_tile_quant(a, ct, r0, r1, act, am);
     } else if ((threadIdx.x & 63) == 0) {
         __hip_atomic_fetch_or(a.epi.status, no_wait ? 2u : 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(a.epi.redo + g * a.ntiles + ct, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(a.epi.redo + mt * a.ntiles + ct, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -238,13 +246,14 @@ __device__ __forceinline__ void decode_finish(const GemmArgs& a, const int g, co
 // workgroup whose own D lies in its own P's expert (possible only with few workgroups, e.g. a
 // partly resident grid).  Such a workgroup does not wait: it leaves P to the fix-up launch and
 // goes on to D, so the waits cannot form a cycle.
+template <int RBM>
 __global__ __launch_bounds__(256, 1) void gmsq_decode_kernel(const GemmArgs a)
 {
     __shared__ int red[3][4][16][64];      // partial sums handed to the wave that owns them (48 KiB)
-    __shared__ float park[4][4][8][2][16]; // the deferred tile's activations (lanes c < 8; 16 KiB)
+    __shared__ float park[4][4][8][RBM][16];  // the deferred tile's activations (lanes c < 8; 8 KiB per row block)
     __shared__ u32 next_t, pend_t;
     const int ntl = a.ntiles;
-    const int count = a.gt.n_groups * ntl;
+    const int count = a.gt.total_mtiles * ntl;
     u32* ticket = a.epi.status + 16;  // the ticket lives in the status block, after the word
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int q = lane >> 4, c = lane & 15;
@@ -253,40 +262,41 @@ __global__ __launch_bounds__(256, 1) void gmsq_decode_kernel(const GemmArgs a)
     int t = (int)next_t;
     __syncthreads();  // every wave has read next_t before thread 0 rewrites it (an empty expert's
                       // iteration has no barrier of its own)
-    int pg = -1, pct = 0, pr0 = 0, pr1 = 0;  // the deferred tile
+    int pm = -1, pct = 0, pr0 = 0, pr1 = 0;  // the deferred tile
     while (t < count) {
         // draw the next ticket now; its result is needed only after this tile
         u32 nt_pending = 0;
         if (threadIdx.x == 0) nt_pending = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int g = t / ntl, ct = t % ntl;
-        const int r0 = g ? a.gt.row_end[g - 1] : 0;
-        const int r1 = a.gt.row_end[g];
-        if (r0 < r1) {
-            float act[2][16];
-            u32 rmax[2];
+        const int mt = t / ntl, ct = t % ntl;
+        const int g = group_of_tile(a.gt, mt);
+        const int r0 = (g ? a.gt.row_end[g - 1] : 0) + (mt - a.gt.tile_start[g]) * 16 * RBM;
+        const int r1 = r0 + 16 * RBM < a.gt.row_end[g] ? r0 + 16 * RBM : a.gt.row_end[g];
+        {
+            float act[RBM][16];
+            u32 rmax[RBM];
             decode_tile_act(a, g, ct, r0, r1, red, act, rmax);
             decode_publish(a, ct, r0, r1, rmax);
-            if (pg >= 0) {
+            if (pm >= 0) {
                 // the ticket drawn at this tile's start (returned by now) decides whether waiting
                 // for the deferred tile could wait for this workgroup itself
                 if (threadIdx.x == 0) pend_t = nt_pending;
                 __syncthreads();
                 const int pend = (int)pend_t;
-                const bool self_dep = pend < count && pend / ntl == pg;
-                float pact[2][16];
+                const bool self_dep = pend < count && pend / ntl == pm;
+                float pact[RBM][16];
 #pragma unroll
-                for (int rb = 0; rb < 2; ++rb)
+                for (int rb = 0; rb < RBM; ++rb)
 #pragma unroll
                     for (int j = 0; j < 16; ++j) pact[rb][j] = c < 8 ? park[wave][q][c & 7][rb][j] : 0.0f;
-                decode_finish(a, pg, pct, pr0, pr1, pact, self_dep);
+                decode_finish(a, pm, pct, pr0, pr1, pact, self_dep);
             }
             if (c < 8) {
 #pragma unroll
-                for (int rb = 0; rb < 2; ++rb)
+                for (int rb = 0; rb < RBM; ++rb)
 #pragma unroll
                     for (int j = 0; j < 16; ++j) park[wave][q][c][rb][j] = act[rb][j];
             }
-            pg = g;
+            pm = mt;
             pct = ct;
             pr0 = r0;
             pr1 = r1;
@@ -296,34 +306,36 @@ __global__ __launch_bounds__(256, 1) void gmsq_decode_kernel(const GemmArgs a)
         t = (int)next_t;
         __syncthreads();  // next_t is rewritten by the next draw
     }
-    if (pg >= 0) {
-        float pact[2][16];
+    if (pm >= 0) {
+        float pact[RBM][16];
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
+        for (int rb = 0; rb < RBM; ++rb)
 #pragma unroll
             for (int j = 0; j < 16; ++j) pact[rb][j] = c < 8 ? park[wave][q][c & 7][rb][j] : 0.0f;
-        decode_finish(a, pg, pct, pr0, pr1, pact);
+        decode_finish(a, pm, pct, pr0, pr1, pact);
     }
 }
 
-// Fix-up launch: tiles marked in redo[g * ntiles + ct], recomputed with the final row maxima.
+// Fix-up launch: tiles marked in redo[mt * ntiles + ct], recomputed with the final row maxima.
+template <int RBM>
 __global__ __launch_bounds__(256, 1) void gmsq_decode_fixup_kernel(const GemmArgs a)
 {
     __shared__ int red[3][4][16][64];
     // no wait timed out in the main launch (status word 0): nothing is marked
     if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(a.epi.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
         return;
-    const int total = a.gt.n_groups * a.ntiles;
+    const int total = a.gt.total_mtiles * a.ntiles;
     for (int t = blockIdx.x; t < total; t += gridDim.x) {
         if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(a.epi.redo + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
             continue;
-        const int g = t / a.ntiles, ct = t % a.ntiles;
-        const int r0 = g ? a.gt.row_end[g - 1] : 0;
-        const int r1 = a.gt.row_end[g];
-        float act[2][16];
-        u32 rmax[2];
+        const int mt = t / a.ntiles, ct = t % a.ntiles;
+        const int g = group_of_tile(a.gt, mt);
+        const int r0 = (g ? a.gt.row_end[g - 1] : 0) + (mt - a.gt.tile_start[g]) * 16 * RBM;
+        const int r1 = r0 + 16 * RBM < a.gt.row_end[g] ? r0 + 16 * RBM : a.gt.row_end[g];
+        float act[RBM][16];
+        u32 rmax[RBM];
         decode_tile_act(a, g, ct, r0, r1, red, act, rmax);
-        float am[2];
+        float am[RBM];
         (void)decode_gather(a, r0, r1, am);  // every slot was written before this launch
         decode_tile_quant(a, ct, r0, r1, act, am);
         __syncthreads();
