@@ -15,14 +15,9 @@
 #include <set>
 #include <utility>
 
-#include "gemm_lds.hpp"
+#include "gemm_tile.hpp"
 
 namespace cb {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef short v4i16 __attribute__((ext_vector_type(4)));
 
 constexpr int kGmmMaxExperts = 64;  // GMM_MAX_E (grouped_matmul_launch.h)
 constexpr int GF_BK = 32;

@@ -80,8 +80,8 @@ inline int check_launch()
 
 // Test hooks (set by cb_set_test_overrides, per thread, until changed): a forced grid for the
 // persistent GEMM kernels (0: the CU count; < 0: persistent launch off), a poll limit for the
-// GroupedMatmulSwigluQuant exchange wait (0: the default), and the GroupedMatmul tile (128 forces
-// the 128 x 128 kernel; 0: automatic).
+// GroupedMatmulSwigluQuant exchange wait (0: the default), and the GEMM tile (1 to 5: a tile of
+// gemm_tile.hpp; 128: the 128 x 128 GroupedMatmul kernel; 0: automatic).
 struct TestOverrides {
     int persistent_grid = 0, exchange_spin_limit = 0, gmm_tile = 0;
 };

@@ -4,6 +4,7 @@
 //   cb_quant_matmul                 (QuantMatmul)
 // plus the status strings.  Each entry point validates in the reference plugin's order, then
 // enqueues its kernels on the caller's stream without any allocation or host synchronisation.
+#include <cmath>
 #include <cstring>
 #include <cstdlib>
 #include <mutex>
@@ -13,6 +14,7 @@
 #include "gmsq_decode.hpp"
 #include "gmsq_prefill.hpp"
 #include "gemm_pf.hpp"
+#include "gemm_tile.hpp"
 
 namespace cb {
 
@@ -118,6 +120,90 @@ static int xcd_split(int ntiles, int64_t E, int64_t tile_row_bytes)
     return 0;
 }
 
+// ---- the dequant GEMM's choice of kernel -------------------------------------------------------
+// Tiles of gemm_tile.hpp.
+using DeqT0 = TileCfg<TileI8, false, 1, 2, 1, 1, 4, 1, 6, 2>;  // 32 x 64
+using DeqT1 = TileCfg<TileI8, false, 2, 4, 1, 1, 4, 1, 3, 2>;  // 64 x 128
+using DeqT2 = TileCfg<TileI8, false, 2, 4, 1, 2, 2, 1, 3, 2>;  // 64 x 256
+using DeqT3 = TileCfg<TileI8, false, 2, 4, 2, 1, 4, 1, 4, 1>;  // 128 x 128, 8 waves
+using DeqT4 = TileCfg<TileI8, false, 2, 4, 2, 2, 2, 1, 6, 1>;  // 128 x 256, 8 waves
+
+template <class C>
+static void launch_deq_tile(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch, hipStream_t st)
+{
+    build_group_table(a.gt, gl, E, C::BM);
+    a.ntiles = (int)((a.N + C::BN - 1) / C::BN);
+    const EpiArgs& e = a.epi;
+    const bool simple = !e.has_offset && e.bias_kind == BIAS_NONE && e.out_bf16;
+    const dim3 grid((unsigned)(a.gt.total_mtiles * a.ntiles), (unsigned)batch);
+    auto go = [&](auto kern) {
+        allow_dynamic_lds((const void*)kern, C::LDS);
+        hipLaunchKernelGGL(kern, grid, dim3(C::NT), C::LDS, st, a);
+    };
+    if (simple) go(tile_gemm_kernel<C, TileDeqEpi<true>>);
+    else go(tile_gemm_kernel<C, TileDeqEpi<false>>);
+}
+
+// Estimated time in us of a BM x BN tile kernel over the call.  A tile alone on its CU takes p us per
+// 128 of K; with a tile on every CU, a round of 256 tiles takes r us per 128 of K plus o us (prologue
+// and epilogue); the bytes the call must move pass at bw TB/s, partly hidden by the multiplications
+// (the two times combine as the root of their squares); f us per call.  The constants are fitted to
+// the measured times below; the 256 x 256 ring core and the skinny kernel (at most 32 rows per
+// group) are candidates like the others, so the rule compares like with like.
+//   us, by rows (dense 7168 x 4096)          us, by rows per expert (256 x 2048 x 7168)
+//                  24    300   1024  2048  4096       8     24    47    96    256
+//   32 x 64       18.3   38     87   165   321       836   912  1257  1971  4750
+//   64 x 128      23.2   24     44    84   161       705   782   829  1054  2019
+//   64 x 256      36     36     41    75   140       680   736   801   988  1764
+//   128 x 128     26     27     35    69   134       921   956  1003  1065  2068
+//   128 x 256     40     42     45    61   118       797   841   907   999  1716
+//   ring          (40)   69     78    98   101       840   839   897   975  1404
+//   skinny        55      -      -     -     -       624
+// With 2048 x 1024 weights 24 rows take 6.0 us (32 x 64) against 16.3 (skinny), 1024 rows 11.3
+// (64 x 128) against 28 (ring); 64 x 768 x 2048 with 200 rows per expert 45 (ring) against 63 (64 x 256).
+struct DeqCand {
+    int bm, bn;
+    double p, r, o, bw, f;
+};
+enum { DEQ_RING = 5, DEQ_SKINNY = 6 };
+static constexpr DeqCand kDeqCand[] = {
+    {32, 64, 0.30, 0.152, 1.5, 5.2, 2.0},   {64, 128, 0.36, 0.31, 2.7, 6.8, 2.0},  {64, 256, 0.58, 0.54, 4.2, 6.55, 2.0},
+    {128, 128, 0.42, 0.486, 6.8, 8.0, 2.0}, {128, 256, 0.64, 0.87, 10.0, 8.0, 2.0}, {256, 256, 1.55, 1.55, 10.0, 12.0, 2.0},
+    {32, 256, 0.85, 0.30, 1.0, 6.3, 3.0},
+};
+
+static int pick_deq(const GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch, int max_rows, bool ring_ok)
+{
+    const double units = (double)((a.K + 127) / 128);
+    int64_t mt[4] = {0, 0, 0, 0}, used = 0, prev = 0;  // row tiles of 32, 64, 128 and 256 rows
+    for (int64_t g = 0; g < E; ++g) {
+        const int64_t rows = gl[g] - prev;
+        for (int j = 0; j < 4; ++j) mt[j] += (rows + (32 << j) - 1) >> (5 + j);
+        used += rows > 0;
+        prev = gl[g];
+    }
+    const double bytes = (double)batch * ((double)used * a.K * a.N + (double)a.M * (a.K + 2 * a.N));
+    double best_t = 0;
+    int best = -1;
+    for (int i = 0; i < (int)(sizeof(kDeqCand) / sizeof(kDeqCand[0])); ++i) {
+        const DeqCand& c = kDeqCand[i];
+        if (i == DEQ_SKINNY && max_rows > kSkinnyMaxRows) continue;
+        if (i == DEQ_RING && !ring_ok) continue;
+        const int64_t tiles = mt[c.bm == 32 ? 0 : c.bm == 64 ? 1 : c.bm == 128 ? 2 : 3] * ((a.N + c.bn - 1) / c.bn) * batch;
+        if (tiles > (1 << 24) && best >= 0) continue;
+        const double rounds = (double)((tiles + 255) / 256);
+        const double full = rounds * (units * c.r + c.o);
+        const double run = full > units * c.p ? full : units * c.p;
+        const double mem = bytes / (c.bw * 1e6);
+        const double t = c.f + std::sqrt(run * run + mem * mem);
+        if (best < 0 || t < best_t) {
+            best = i;
+            best_t = t;
+        }
+    }
+    return best;
+}
+
 template <int EPI>
 static void launch_gemm(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch, bool fast, hipStream_t st)
 {
@@ -135,6 +221,23 @@ static void launch_gemm(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch
         else
             hipLaunchKernelGGL(generic_dequant_kernel, grid, dim3(256), 0, st, a);
         return;
+    }
+    if constexpr (EPI == EPI_DEQUANT) {
+        const int64_t rows = a.gt.max_rows;
+        // 32-bit offsets within a tile's activation and output rows
+        const bool tile_ok = 128 * a.K < 0x7fffffffLL && 256 * Ncols < 0x7fffffffLL && batch <= 65535;
+        int pick = -1;
+        if (tile_ok && g_overrides.gmm_tile > 0 && g_overrides.gmm_tile <= 5) pick = g_overrides.gmm_tile - 1;  // test hook
+        else if (tile_ok && g_overrides.persistent_grid == 0)
+            pick = pick_deq(a, gl, E, batch, (int)rows, a.K >= 4 * PfCfg::BK || batch > 1);
+        switch (pick) {
+            case 0: launch_deq_tile<DeqT0>(a, gl, E, batch, st); return;
+            case 1: launch_deq_tile<DeqT1>(a, gl, E, batch, st); return;
+            case 2: launch_deq_tile<DeqT2>(a, gl, E, batch, st); return;
+            case 3: launch_deq_tile<DeqT3>(a, gl, E, batch, st); return;
+            case 4: launch_deq_tile<DeqT4>(a, gl, E, batch, st); return;
+            default: break;  // the skinny kernel or the 256 x 256 cores below
+        }
     }
     if (a.gt.max_rows <= kSkinnyMaxRows) {
         a.ntiles = (int)((Ncols + 255) / 256);
@@ -163,9 +266,9 @@ static void launch_gemm(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch
             const bool simple = !e.has_offset && e.bias_kind == BIAS_NONE && e.out_bf16;
             const void* kern = simple ? (const void*)gpf_dequant_kernel<true> : (const void*)gpf_dequant_kernel<false>;
             allow_dynamic_lds(kern, kGpfLds);
-            // the block map's valid slots are spread over each round of 256: launch the whole grid
-            const bool bm = gpf_block_map(a.gt.total_mtiles, a.ntiles);
-            const dim3 grid((unsigned)(bm || blocks > pg ? pg : blocks));
+            // both launch orders spread the valid slots over up to a round of 256: launch the whole
+            // grid (a grid of `blocks` workgroups walked several tiles each while others had none)
+            const dim3 grid((unsigned)pg);
             if (simple) hipLaunchKernelGGL(gpf_dequant_kernel<true>, grid, dim3(256), kGpfLds, st, a);
             else hipLaunchKernelGGL(gpf_dequant_kernel<false>, grid, dim3(256), kGpfLds, st, a);
             return;

@@ -1,0 +1,81 @@
+"""GPU parity of the tiled GEMMs between the skinny and the 256 x 256 kernels (QuantMatmul and the
+int8 grouped down-projection), each tile forced in turn through the library's test override: row
+counts around the 32-row fragments and the tile edges, partial column tiles (N off every tile
+width), K of one 16-byte chunk, below, at and past a stage and the ring's depth, ragged and empty
+groups, every dequant flag and a batch.  The int32 sums are exact and the dequant chain rounds in
+the oracle's order, so the bar is bit equality."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+def _i8(rng, *shape):
+    return rng.integers(-127, 128, size=shape, dtype=np.int8)
+
+
+def _dev(*arrays):
+    return [torch.from_numpy(a).to(DEV) for a in arrays]
+
+
+def bits16(t):
+    return t.contiguous().view(torch.int16).cpu().numpy().view(np.uint16)
+
+
+@pytest.fixture(params=[1, 2, 3, 4, 5])  # 32 x 64, 64 x 128, 64 x 256, 128 x 128, 128 x 256
+def tile(request, overrides):
+    overrides(gmm_tile=request.param)
+    return request.param
+
+
+GROUPED = [
+    # (counts, K, N)
+    ([1, 0, 31, 33], 16, 16),
+    ([64, 65, 0, 127], 144, 272),
+    ([129, 2], 1040, 528),
+    ([300, 0, 0, 7], 2048, 80),
+]
+
+
+@pytest.mark.parametrize("counts,K,N", GROUPED)
+def test_tile_grouped(cb, orc, tile, counts, K, N):
+    rng = np.random.default_rng(K + N)
+    E, M = len(counts), sum(counts)
+    x, w = _i8(rng, M, K), _i8(rng, E, K, N)
+    ws = rng.uniform(0.001, 0.01, (E, N)).astype(np.float32)
+    xs = rng.uniform(0.005, 0.02, M).astype(np.float32)
+    gl = np.cumsum(counts)
+    out = cb.grouped_matmul_quant(*_dev(x, w, ws, xs), gl.tolist())
+    np.testing.assert_array_equal(bits16(out), orc.grouped_matmul_quant(x, w, ws, xs, gl))
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 256, 64), (32, 400, 144), (200, 640, 496)])
+@pytest.mark.parametrize("flags", ["plain", "i32", "full", "perchan_off"])
+def test_tile_quant_matmul(cb, orc, tile, M, K, N, flags):
+    rng = np.random.default_rng(M + K)
+    x1, x2 = _i8(rng, M, K), _i8(rng, K, N)
+    scale = rng.uniform(0.001, 0.01, 1 if flags == "perchan_off" else N).astype(np.float32)
+    pt = None if flags == "i32" else rng.uniform(0.005, 0.02, M).astype(np.float32)
+    off = rng.uniform(-1, 1, N).astype(np.float32) if flags == "full" else None
+    bias = {"i32": rng.integers(-5000, 5000, N, dtype=np.int32), "full": rng.normal(size=N).astype(np.float32)}.get(flags)
+    dt = "bfloat16" if flags in ("plain", "full") else "float16"
+    opt = lambda a: None if a is None else torch.from_numpy(a).to(DEV)
+    out = cb.quant_matmul(*_dev(x1, x2, scale), offset=opt(off), pertoken_scale=opt(pt), bias=opt(bias), output_dtype=dt)
+    ref = orc.quant_matmul(x1, x2, scale, offset=off, pertoken=pt, bias=bias,
+                           bias_dtype="i32" if flags == "i32" else "f32", out_dtype="bf16" if dt == "bfloat16" else "f16")
+    np.testing.assert_array_equal(bits16(out), ref)
+
+
+def test_tile_batched(cb, tile):
+    rng = np.random.default_rng(3)
+    x1, x2 = _i8(rng, 3, 70, 272), _i8(rng, 3, 272, 144)
+    scale = rng.uniform(0.001, 0.01, 144).astype(np.float32)
+    bias = rng.integers(-5000, 5000, (3, 1, 144), dtype=np.int32)
+    d = _dev(x1, x2, scale, bias)
+    out = cb.quant_matmul(*d[:3], bias=d[3], output_dtype="bfloat16")
+    acc = np.matmul(x1.astype(np.int64), x2.astype(np.int64)).astype(np.float32) + bias.astype(np.float32)
+    ref = torch.from_numpy(acc * scale).to(torch.bfloat16)
+    assert torch.equal(out.cpu(), ref)
