@@ -88,6 +88,9 @@ struct GemmArgs {
     GroupTable gt;
 };
 
+// The dequant GEMM on tile 0 to 4 of deq_tile.hip; false for any other number.
+bool launch_deq_tile(int tile, GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch, hipStream_t st);
+
 // Source row of routed row r: r itself, or row_index[r]; -1 when the index lies outside
 // [0, x_rows) (such a row reads as zeros with scale 0).
 __device__ __forceinline__ int src_row(const GemmArgs& a, int r)

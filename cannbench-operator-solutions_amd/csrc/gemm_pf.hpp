@@ -20,7 +20,7 @@
 #pragma once
 
 #include "gmsq_prefill.hpp"
-#include "gemm_tile.hpp"
+#include "quad16.hpp"
 
 namespace cb {
 

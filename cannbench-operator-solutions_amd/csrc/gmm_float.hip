@@ -11,9 +11,6 @@
 // (K or N not a multiple of 8, misaligned operands, 32-bit offsets exceeded) take a plain fp32 loop.
 #include <cstdlib>
 #include <cstring>
-#include <mutex>
-#include <set>
-#include <utility>
 
 #include "gemm_tile.hpp"
 
@@ -439,18 +436,6 @@ __global__ __launch_bounds__(256) void gmm_generic_kernel(const GmmFArgs a)
 // A test override of 128 selects the 128 x 128 register-staged kernel for every fp16/bf16 shape (it
 // is otherwise taken only where a 256-row block of x or y passes 2 GiB).
 static bool gmm_lds_enabled() { return g_overrides.gmm_tile != 128; }
-
-// Raise a kernel's dynamic LDS limit once per (kernel, device).
-static void set_dynamic_lds_once(const void* kern, int bytes)
-{
-    static std::mutex mu;
-    static std::set<std::pair<const void*, int>> done;
-    int dev = -1;
-    (void)hipGetDevice(&dev);
-    std::lock_guard<std::mutex> lock(mu);
-    if (done.insert({kern, dev}).second)
-        (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-}
 
 }  // namespace cb
 

@@ -87,6 +87,10 @@ struct TestOverrides {
 };
 extern thread_local TestOverrides g_overrides;
 
+// Raise a kernel's dynamic LDS limit once per (kernel, device): the attribute belongs to the kernel as
+// loaded on the current device, so a process driving several GPUs sets it on each.
+void set_dynamic_lds_once(const void* kern, int bytes);
+
 // Optional per-thread instrumentation: events recorded around the next main kernel launch of an
 // operator (set by cb_set_kernel_timing, consumed and cleared by that launch).
 struct KernelTiming {

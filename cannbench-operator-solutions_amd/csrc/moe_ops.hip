@@ -14,7 +14,6 @@
 #include "gmsq_decode.hpp"
 #include "gmsq_prefill.hpp"
 #include "gemm_pf.hpp"
-#include "gemm_tile.hpp"
 
 namespace cb {
 
@@ -90,9 +89,7 @@ static int persistent_grid()
 // that gives up is recomputed by the fix-up launch, so the limit bounds the wait, not correctness.
 static constexpr int kExchangeSpins = 1 << 20;
 
-// Raise a kernel's dynamic LDS limit once per (kernel, device): the attribute belongs to the
-// kernel as loaded on the current device, so a process driving several GPUs sets it on each.
-static void allow_dynamic_lds(const void* kern, int bytes)
+void set_dynamic_lds_once(const void* kern, int bytes)
 {
     static std::mutex mu;
     static std::set<std::pair<const void*, int>> done;
@@ -121,29 +118,6 @@ static int xcd_split(int ntiles, int64_t E, int64_t tile_row_bytes)
 }
 
 // ---- the dequant GEMM's choice of kernel -------------------------------------------------------
-// Tiles of gemm_tile.hpp.
-using DeqT0 = TileCfg<TileI8, false, 1, 2, 1, 1, 4, 1, 6, 2>;  // 32 x 64
-using DeqT1 = TileCfg<TileI8, false, 2, 4, 1, 1, 4, 1, 3, 2>;  // 64 x 128
-using DeqT2 = TileCfg<TileI8, false, 2, 4, 1, 2, 2, 1, 3, 2>;  // 64 x 256
-using DeqT3 = TileCfg<TileI8, false, 2, 4, 2, 1, 4, 1, 4, 1>;  // 128 x 128, 8 waves
-using DeqT4 = TileCfg<TileI8, false, 2, 4, 2, 2, 2, 1, 6, 1>;  // 128 x 256, 8 waves
-
-template <class C>
-static void launch_deq_tile(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch, hipStream_t st)
-{
-    build_group_table(a.gt, gl, E, C::BM);
-    a.ntiles = (int)((a.N + C::BN - 1) / C::BN);
-    const EpiArgs& e = a.epi;
-    const bool simple = !e.has_offset && e.bias_kind == BIAS_NONE && e.out_bf16;
-    const dim3 grid((unsigned)(a.gt.total_mtiles * a.ntiles), (unsigned)batch);
-    auto go = [&](auto kern) {
-        allow_dynamic_lds((const void*)kern, C::LDS);
-        hipLaunchKernelGGL(kern, grid, dim3(C::NT), C::LDS, st, a);
-    };
-    if (simple) go(tile_gemm_kernel<C, TileDeqEpi<true>>);
-    else go(tile_gemm_kernel<C, TileDeqEpi<false>>);
-}
-
 // Estimated time in us of a BM x BN tile kernel over the call.  A tile alone on its CU takes p us per
 // 128 of K; with a tile on every CU, a round of 256 tiles takes r us per 128 of K plus o us (prologue
 // and epilogue); the bytes the call must move pass at bw TB/s, partly hidden by the multiplications
@@ -230,14 +204,8 @@ static void launch_gemm(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch
         if (tile_ok && g_overrides.gmm_tile > 0 && g_overrides.gmm_tile <= 5) pick = g_overrides.gmm_tile - 1;  // test hook
         else if (tile_ok && g_overrides.persistent_grid == 0)
             pick = pick_deq(a, gl, E, batch, (int)rows, a.K >= 4 * PfCfg::BK || batch > 1);
-        switch (pick) {
-            case 0: launch_deq_tile<DeqT0>(a, gl, E, batch, st); return;
-            case 1: launch_deq_tile<DeqT1>(a, gl, E, batch, st); return;
-            case 2: launch_deq_tile<DeqT2>(a, gl, E, batch, st); return;
-            case 3: launch_deq_tile<DeqT3>(a, gl, E, batch, st); return;
-            case 4: launch_deq_tile<DeqT4>(a, gl, E, batch, st); return;
-            default: break;  // the skinny kernel or the 256 x 256 cores below
-        }
+        // otherwise the skinny kernel or the 256 x 256 cores below
+        if (launch_deq_tile(pick, a, gl, E, batch, st)) return;
     }
     if (a.gt.max_rows <= kSkinnyMaxRows) {
         a.ntiles = (int)((Ncols + 255) / 256);
@@ -265,7 +233,7 @@ static void launch_gemm(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch
             const EpiArgs& e = a.epi;
             const bool simple = !e.has_offset && e.bias_kind == BIAS_NONE && e.out_bf16;
             const void* kern = simple ? (const void*)gpf_dequant_kernel<true> : (const void*)gpf_dequant_kernel<false>;
-            allow_dynamic_lds(kern, kGpfLds);
+            set_dynamic_lds_once(kern, kGpfLds);
             // both launch orders spread the valid slots over up to a round of 256: launch the whole
             // grid (a grid of `blocks` workgroups walked several tiles each while others had none)
             const dim3 grid((unsigned)pg);
@@ -282,12 +250,12 @@ static void launch_gemm(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch
         Cfg::BM * Ncols * 4 < 0x7fffffffLL) {
         auto kern = lds_gemm_persistent_kernel<EPI, kLdsWM, kLdsWN, kLdsStages, kLdsBK>;
         constexpr int lds = Cfg::CONT_LDS_BYTES;  // the ring and two row-scale slots
-        allow_dynamic_lds((const void*)kern, lds);
+        set_dynamic_lds_once((const void*)kern, lds);
         hipLaunchKernelGGL(kern, dim3((unsigned)pg), dim3(Cfg::NT), lds, st, a);
         return;
     }
     auto kern = lds_gemm_kernel<EPI, kLdsWM, kLdsWN, kLdsStages, kLdsBK>;
-    allow_dynamic_lds((const void*)kern, Cfg::LDS_BYTES);
+    set_dynamic_lds_once((const void*)kern, Cfg::LDS_BYTES);
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks, (unsigned)batch), dim3(Cfg::NT), Cfg::LDS_BYTES, st, a);
 }
 
@@ -436,8 +404,8 @@ static int gmsq_impl(const int8_t* x, int64_t x_rows, const int32_t* row_index, 
         if (grid >= ntl && resident >= 1 && a.gt.total_mtiles + 2 <= ws.n_arrive) {
             a.ntiles = ntl;
             clear_ws((int64_t)a.gt.total_mtiles * ntl);
-            allow_dynamic_lds(main_k, kPfLds);
-            allow_dynamic_lds(fix_k, kPfLds);
+            set_dynamic_lds_once(main_k, kPfLds);
+            set_dynamic_lds_once(fix_k, kPfLds);
             const int tiles = a.gt.total_mtiles * ntl;
             const dim3 fix_grid((unsigned)(tiles < 256 ? tiles : 256));
             {
