@@ -4,10 +4,10 @@
 // (operators/groupedmatmul/csrc/ops/grouped_matmul/op_plugin/grouped_matmul_plugin.cpp:14-17,
 // 116-183; op_kernel/grouped_matmul_kernel.cpp:15-17, 111-150).
 //
-// 16-bit inputs run on v_mfma_f32_32x32x16_{f16,bf16}: 128 x 128 output tiles (4 waves of 64 x 64),
-// 32-deep K stages double-buffered in LDS with both operands stored K-contiguous (the weight is
-// transposed on its way into LDS when it arrives N-contiguous), fp32 accumulation, the bias added
-// in fp32, one round-to-nearest-even narrowing.  fp32 inputs and shapes off the vector path
+// 16-bit inputs run on v_mfma_f32_32x32x16_{f16,bf16} through the tiles of gemm_tile.hpp (32 x 64 to
+// 256 x 256, chosen by pick_gmm), fp32 accumulation, the bias added in fp32, one
+// round-to-nearest-even narrowing.  Rows or outputs past 32-bit offsets take a 128 x 128
+// register-staged kernel.  fp32 inputs and shapes off the vector path
 // (K or N not a multiple of 8, misaligned operands, 32-bit offsets exceeded) take a plain fp32 loop.
 #include <cstdlib>
 #include <cstring>
@@ -224,193 +224,38 @@ __global__ __launch_bounds__(64 * WM * WN, 64 * WM * WN > 256 ? 1 : 2) void gmm_
     }
 }
 
-// 256 x 256 tiles on the int8 LDS core's structure: 8 waves (4 x 2) of 64 x 128, 64-deep stages
-// (128 bytes of every operand row) DMA'd from global memory straight into a 2-stage LDS ring
-// (buffer_load ... lds), one stage in flight while the other is multiplied.
-//   x rows and a [N][K] weight: K-contiguous rows of 128 bytes, 16-byte chunks XOR-swizzled by
-//   (row >> 1) & 7 (as the int8 core's A), fragments read with ds_read_b128.
-//   a [K][N] weight: 64 rows of 256 columns (512 bytes), 16-byte chunks XOR-swizzled by 2 (k % 4);
-//   fragments read with ds_read_b64_tr_b16: in each 16-lane group, lane s addresses row
-//   k0 + s / 4, columns nb + 4 (s % 4) .. + 3, and lane j receives k0 .. k0 + 3 of column nb + j.
-// Chunks past K or N point outside their buffer resource and read zeros.
-constexpr int GL_BM = 256, GL_BN = 256, GL_BK = 64, GL_WN = 2, GL_NT = 512;  // 4 x 2 waves
-constexpr int GL_ROWB = GL_BK * 2;                 // bytes per K-contiguous row and stage
-constexpr int GL_A_BYTES = GL_BM * GL_ROWB;        // 32 KB
-constexpr int GL_B_BYTES = GL_BN * GL_ROWB;        // 32 KB either layout
-constexpr int GL_STAGE = GL_A_BYTES + GL_B_BYTES;
-constexpr int GL_ISSUE = (GL_A_BYTES + GL_B_BYTES) / 16 / GL_NT;  // DMAs per thread per stage (8)
-
-__device__ __forceinline__ int gl_swz(int r) { return (r >> 1) & 7; }
-
-template <bool BF16, bool TRANS>
-__global__ __launch_bounds__(GL_NT, 1) void gmm_lds_kernel(const GmmFArgs a)
-{
-    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-    constexpr int GROUP_M = 4;
-    const int pid = blockIdx.x;
-    const int T_m = a.gt.total_mtiles, T_n = a.ntiles;
-    const int per_group = GROUP_M * T_n;
-    const int first_m = (pid / per_group) * GROUP_M;
-    const int gsz = (T_m - first_m) < GROUP_M ? (T_m - first_m) : GROUP_M;
-    const int mt = first_m + (pid % per_group) % gsz;
-    const int nt = (pid % per_group) / gsz;
-    const int g = group_of_tile(a.gt, mt);
-    const int rs = g ? a.gt.row_end[g - 1] : 0;
-    const int r1 = a.gt.row_end[g];
-    const int m0 = rs + (mt - a.gt.tile_start[g]) * GL_BM;
-    const int vrows = r1 - m0;
-    const int n0 = nt * GL_BN;
-    const int64_t K = a.K, N = a.N;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / GL_WN, wn = wave % GL_WN;
-    const uint32_t lds_base = (uint32_t)(uintptr_t)(CB_LDS uint8_t*)smem;
-
-    const __amdgpu_buffer_rsrc_t ares = make_rsrc((const uint16_t*)a.x + (int64_t)m0 * K,
-                                                     (uint32_t)((vrows < GL_BM ? vrows : GL_BM) * K * 2));
-    const __amdgpu_buffer_rsrc_t bres = make_rsrc((const uint16_t*)a.w + (int64_t)g * K * N, (uint32_t)(K * N * 2));
-    // per DMA i: the element offset of the chunk at k = 0 (or -1: nothing to fetch) and its k start
-    int64_t aoff[4], boff[4];
-    int akq[4], bk[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int cid = (i * 8 + wave) * 64 + lane;  // lane-linear 16-byte chunk of the stage
-        const int row = cid >> 3, pos = cid & 7;
-        const int q = pos ^ gl_swz(row);
-        akq[i] = q * 8;
-        aoff[i] = row < vrows ? (int64_t)row * K + q * 8 : -1;
-        if constexpr (TRANS) {
-            bk[i] = q * 8;
-            boff[i] = n0 + row < N ? (int64_t)(n0 + row) * K + q * 8 : -1;
-        } else {
-            const int krow = cid >> 5, cpos = cid & 31;
-            const int c = cpos ^ (2 * (krow & 3));  // logical 8-column chunk
-            bk[i] = krow;
-            boff[i] = n0 + c * 8 < N ? (int64_t)krow * N + n0 + c * 8 : -1;
-        }
-    }
-    const int nk = (int)((K + GL_BK - 1) / GL_BK);
-    auto issue = [&](int kt) {
-        const uint32_t sa = lds_base + (uint32_t)((kt & 1) * GL_STAGE);
-        const int k0 = kt * GL_BK;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const bool ok = aoff[i] >= 0 && k0 + akq[i] < K;
-            dma16(ares, ok ? (uint32_t)((aoff[i] + k0) * 2) : 0x80000000u,
-                  __builtin_amdgcn_readfirstlane(sa + (uint32_t)((i * 8 + wave) * 1024)));
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            bool ok;
-            int64_t off;
-            if constexpr (TRANS) {
-                ok = boff[i] >= 0 && k0 + bk[i] < K;
-                off = boff[i] + k0;
-            } else {
-                ok = boff[i] >= 0 && k0 + bk[i] < K;
-                off = boff[i] + (int64_t)k0 * N;
-            }
-            dma16(bres, ok ? (uint32_t)(off * 2) : 0x80000000u,
-                  __builtin_amdgcn_readfirstlane(sa + GL_A_BYTES + (uint32_t)((i * 8 + wave) * 1024)));
-        }
+// Epilogue of the tiled GEMM (gemm_tile.hpp): the bias added in fp32, one narrowing.
+template <bool BF16>
+struct GmmTileEpi {
+    using Args = GmmFArgs;
+    struct Pre {
+        float bias;
     };
-
-    f32x16 acc[2][4];
-#pragma unroll
-    for (int fm = 0; fm < 2; ++fm)
-#pragma unroll
-        for (int fn = 0; fn < 4; ++fn)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[fm][fn][r] = 0.0f;
-
-    issue(0);
-    issue(1);
-    for (int kt = 0; kt < nk; ++kt) {
-        wait_vmcnt_barrier<GL_ISSUE>();  // stage kt has landed (stage kt + 1 may stay in flight)
-        const CB_LDS uint8_t* st = (const CB_LDS uint8_t*)smem + (kt & 1) * GL_STAGE;
-#pragma unroll
-        for (int ks = 0; ks < GL_BK / 16; ++ks) {
-            uint4 af[2], bfr[4];
-            const int q = 2 * ks + (lane >> 5);
-#pragma unroll
-            for (int fm = 0; fm < 2; ++fm) {
-                const int r = wm * 64 + fm * 32 + (lane & 31);
-                af[fm] = __builtin_bit_cast(uint4, *(const CB_LDS v4i*)(st + r * GL_ROWB + ((q ^ gl_swz(r)) << 4)));
-            }
-#pragma unroll
-            for (int fn = 0; fn < 4; ++fn) {
-                if constexpr (TRANS) {
-                    const int r = wn * 128 + fn * 32 + (lane & 31);
-                    bfr[fn] = __builtin_bit_cast(uint4, *(const CB_LDS v4i*)(st + GL_A_BYTES + r * GL_ROWB + ((q ^ gl_swz(r)) << 4)));
-                } else {
-                    const int grp = lane >> 4, s = lane & 15;
-                    const int nb = wn * 128 + fn * 32 + 16 * (grp & 1);
-                    const int col = nb + 4 * (s & 3);
-                    u32 w[4];
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const int k = ks * 16 + 8 * (grp >> 1) + 4 * h + (s >> 2);
-                        const int chunk = (col >> 3) ^ (2 * (k & 3));
-                        const v4i16 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                            (CB_LDS v4i16*)(st + GL_A_BYTES + k * (GL_BN * 2) + chunk * 16 + (col & 7) * 2));
-                        w[2 * h] = (u32)(uint16_t)v[0] | ((u32)(uint16_t)v[1] << 16);
-                        w[2 * h + 1] = (u32)(uint16_t)v[2] | ((u32)(uint16_t)v[3] << 16);
-                    }
-                    bfr[fn] = make_uint4(w[0], w[1], w[2], w[3]);
-                }
-            }
-#pragma unroll
-            for (int fm = 0; fm < 2; ++fm)
-#pragma unroll
-                for (int fn = 0; fn < 4; ++fn) {
-                    if constexpr (BF16)
-                        acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            __builtin_bit_cast(bf16x8, af[fm]), __builtin_bit_cast(bf16x8, bfr[fn]), acc[fm][fn], 0, 0, 0);
-                    else
-                        acc[fm][fn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                            __builtin_bit_cast(f16x8, af[fm]), __builtin_bit_cast(f16x8, bfr[fn]), acc[fm][fn], 0, 0, 0);
-                }
-        }
-        // every wave is done with this buffer before the DMA of stage kt + 2 overwrites it
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        issue(kt + 2);  // past K: fetches nothing
+    __device__ static __forceinline__ const uint8_t* x_base(const Args& a, const int) { return (const uint8_t*)a.x; }
+    __device__ static __forceinline__ const uint8_t* w_base(const Args& a, const int g, const int)
+    {
+        return (const uint8_t*)a.w + (int64_t)g * a.K * a.N * 2;
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-
-    // Epilogue.  32x32 C layout: lane l holds column l % 32, rows 8 (r / 4) + 4 (l / 32) + r % 4.
-    // Rows r and r + 1 of a lane pair (l, l ^ 1) are swapped so that each lane stores two adjacent
-    // columns of one row as one dword: the even lane row r, columns (c, c + 1), the odd lane row
-    // r + 1, columns (c - 1, c).  Rows past the group's end fall outside the resource and are dropped.
-    const __amdgpu_buffer_rsrc_t ores = make_rsrc((uint16_t*)a.y + (int64_t)m0 * N,
-                                                  (uint32_t)((vrows < GL_BM ? vrows : GL_BM) * N * 2));
-    const bool odd = lane & 1;
-    float bv[4];
-    uint32_t coff[4];
-#pragma unroll
-    for (int fn = 0; fn < 4; ++fn) {
-        const int64_t col = n0 + wn * 128 + fn * 32 + (lane & 31);
-        bv[fn] = a.bias_dt ? gf_load(a.bias, a.bias_dt, (int64_t)g * N + (col < N ? col : 0)) : 0.0f;
-        coff[fn] = col < N ? (uint32_t)(col & ~(int64_t)1) * 2u : 0x80000000u;
+    __device__ static __forceinline__ uint16_t* out_base(const Args& a, const int) { return (uint16_t*)a.y; }
+    // thread tid: the bias of tile column tid (columns past N repeat the last)
+    __device__ static __forceinline__ Pre load(const Args& a, const TileAt& t, const int, const int n0, const int, const int tid)
+    {
+        const int64_t col = (int64_t)n0 + tid < a.N ? (int64_t)n0 + tid : a.N - 1;
+        return Pre{a.bias_dt ? gf_load(a.bias, a.bias_dt, (int64_t)t.g * a.N + col) : 0.0f};
     }
+    __device__ static __forceinline__ void put(const Pre& p, CB_LDS float* sc, const int bm, const int bn, const int tid)
+    {
+        if (tid < bn) sc[bm + tid] = p.bias;
+    }
+    __device__ static __forceinline__ void narrow(const Args&, const CB_LDS float* sc, const int bm, const int, const int,
+                                                  const int col, const float (&v)[8], u32 (&p)[4])
+    {
+        const float b = sc[bm + col];
 #pragma unroll
-    for (int fm = 0; fm < 2; ++fm)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-            const int lrow = wm * 64 + fm * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);  // rows lrow, lrow + 1
-            const uint32_t roff = (uint32_t)(lrow + (odd ? 1 : 0)) * (uint32_t)N * 2u;
-#pragma unroll
-            for (int fn = 0; fn < 4; ++fn) {
-                const float v0 = acc[fm][fn][r] + bv[fn], v1 = acc[fm][fn][r + 1] + bv[fn];
-                const uint32_t h0 = BF16 ? f32_to_bf16_hw(v0) : f32_to_f16(v0);
-                const uint32_t h1 = BF16 ? f32_to_bf16_hw(v1) : f32_to_f16(v1);
-                const uint32_t p = h0 | (h1 << 16);
-                // partner lane's pair (quad_perm [1, 0, 3, 2])
-                const uint32_t q = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p, 0xB1, 0xF, 0xF, false);
-                const uint32_t w = odd ? ((q >> 16) | (p & 0xffff0000u)) : ((p & 0xffffu) | (q << 16));
-                __builtin_amdgcn_raw_buffer_store_b32(w, ores, roff + coff[fn], 0, 0);
-            }
-        }
-}
+        for (int i = 0; i < 4; ++i)
+            p[i] = BF16 ? pack_bf16x2(v[2 * i] + b, v[2 * i + 1] + b) : pack_f16x2(v[2 * i] + b, v[2 * i + 1] + b);
+    }
+};
 
 // Any dtype and layout: one output element per thread iteration (grid-stride), fp32 accumulation
 // in k order, the bias added in fp32, one narrowing to the output dtype.
@@ -433,9 +278,86 @@ __global__ __launch_bounds__(256) void gmm_generic_kernel(const GmmFArgs a)
     }
 }
 
-// A test override of 128 selects the 128 x 128 register-staged kernel for every fp16/bf16 shape (it
-// is otherwise taken only where a 256-row block of x or y passes 2 GiB).
-static bool gmm_lds_enabled() { return g_overrides.gmm_tile != 128; }
+template <template <class, bool> class Cfg>
+static void launch_gmm_tile(GmmFArgs& a, const int64_t* gl, int64_t E, hipStream_t st)
+{
+    using C0 = Cfg<TileBF16, false>;
+    build_group_table(a.gt, gl, E, C0::BM);
+    a.ntiles = (int)((a.N + C0::BN - 1) / C0::BN);
+    const dim3 grid((unsigned)(a.gt.total_mtiles * a.ntiles));
+    auto go = [&](auto cfg, auto epi) {
+        using C = decltype(cfg);
+        auto kern = tile_gemm_kernel<C, decltype(epi)>;
+        set_dynamic_lds_once((const void*)kern, C::LDS);
+        hipLaunchKernelGGL(kern, grid, dim3(C::NT), C::LDS, st, a);
+    };
+    const bool bf = a.x_dt == CB_DT_BFLOAT16;
+    if (bf && a.trans) go(Cfg<TileBF16, true>{}, GmmTileEpi<true>{});
+    else if (bf) go(Cfg<TileBF16, false>{}, GmmTileEpi<true>{});
+    else if (a.trans) go(Cfg<TileF16, true>{}, GmmTileEpi<false>{});
+    else go(Cfg<TileF16, false>{}, GmmTileEpi<false>{});
+}
+
+template <class OP, bool BT> using GmmT0 = TileCfg<OP, BT, 1, 2, 1, 1, 4, 1, 6, 2>;  // 32 x 64
+template <class OP, bool BT> using GmmT1 = TileCfg<OP, BT, 2, 4, 1, 1, 4, 1, 3, 2>;  // 64 x 128
+template <class OP, bool BT> using GmmT2 = TileCfg<OP, BT, 2, 4, 1, 2, 2, 1, 3, 2>;  // 64 x 256
+template <class OP, bool BT> using GmmT3 = TileCfg<OP, BT, 2, 4, 2, 1, 4, 1, 4, 1>;  // 128 x 128, 8 waves
+template <class OP, bool BT> using GmmT4 = TileCfg<OP, BT, 2, 4, 2, 2, 2, 2, 3, 1>;  // 128 x 256, 8 waves
+template <class OP, bool BT> using GmmT5 = TileCfg<OP, BT, 2, 4, 4, 2, 1, 2, 4, 1>;  // 256 x 256, 8 waves
+
+// Estimated time of each tile over the call, in the terms of the int8 rule (moe_ops.hip: us per 128
+// bytes of K for a tile alone and in a full round of 256, us per round), combined with the bytes at
+// bw TB/s; the least is taken.  The choice does not look at the weight layout, so that [K][N] and
+// [N][K] storage of the same weights are summed in the same order and agree bit for bit.  Measured
+// us, 64 experts of 4096 x 4096 bf16, [K][N] / [N][K] weights (first: the 256 x 256 double-buffered
+// kernel these replace):
+//   rows per expert     8          24         64         128        256         512
+//   (replaced)       479 / 510  484 / 527  514 / 538  544 / 566  871 / 862  1377 / 1352
+//   32 x 64          377 / 362  419 / 389  583 / 575  855 / 866    -           -
+//   64 x 128         374 / 363  388 / 372  467 / 443  601 / 605  936 / 946     -
+//   64 x 256         346 / 375  354 / 388  444 / 494  540 / 635  870 / 1017    -
+//   128 x 128        402 / 384  409 / 395  437 / 414  554 / 549  845 / 837  1430 / 1401
+//   128 x 256        355 / 372     -       384 / 394  495 / 490  750 / 764  1234 / 1226
+//   256 x 256        409 / 425     -       457 / 485  487 / 544  801 / 875  1241 / 1323
+// 8 experts of 2048 x 1536, 8 rows each: 53 -> 13.6 (32 x 64); 1024 rows each: 69 -> 62 (256 x 256).
+struct GmmCand {
+    int bm, bn;
+    double p, r, o, bw;
+};
+static constexpr GmmCand kGmmCand[] = {
+    {32, 64, 0.30, 0.152, 1.5, 6.0},  {64, 128, 0.36, 0.34, 2.7, 6.0}, {64, 256, 0.58, 0.66, 5.0, 6.2},
+    {128, 128, 0.42, 0.51, 6.8, 6.2}, {128, 256, 0.90, 0.92, 9.0, 6.2}, {256, 256, 1.30, 1.75, 8.0, 6.2},
+};
+
+static int pick_gmm(const GmmFArgs& a, const int64_t* gl, int64_t E)
+{
+    const double units = (double)((a.K + 63) / 64);
+    int64_t mt[4] = {0, 0, 0, 0}, used = 0, prev = 0;  // row tiles of 32, 64, 128 and 256 rows
+    for (int64_t g = 0; g < E; ++g) {
+        const int64_t rows = gl[g] - prev;
+        for (int j = 0; j < 4; ++j) mt[j] += (rows + (32 << j) - 1) >> (5 + j);
+        used += rows > 0;
+        prev = gl[g];
+    }
+    const double bytes = 2.0 * ((double)used * a.K * a.N + (double)a.M * (a.K + a.N));
+    double best_t = 0;
+    int best = -1;
+    for (int i = 0; i < (int)(sizeof(kGmmCand) / sizeof(kGmmCand[0])); ++i) {
+        const GmmCand& c = kGmmCand[i];
+        const int64_t tiles = mt[c.bm == 32 ? 0 : c.bm == 64 ? 1 : c.bm == 128 ? 2 : 3] * ((a.N + c.bn - 1) / c.bn);
+        if (tiles > (1 << 30)) continue;
+        const double rounds = (double)((tiles + 255) / 256);
+        const double full = rounds * (units * c.r + c.o), alone = units * c.p + c.o;
+        const double run = tiles >= 256 || full < alone ? full : alone + (full - alone) * (double)tiles / 256;
+        const double mem = bytes / (c.bw * 1e6);
+        const double t = run * run * run * run + mem * mem * mem * mem;
+        if (best < 0 || t < best_t) {
+            best = i;
+            best_t = t;
+        }
+    }
+    return best;
+}
 
 }  // namespace cb
 
@@ -478,20 +400,20 @@ extern "C" int cb_grouped_matmul(const void* x, const void* weight, const void* 
     const bool mfma = x_dtype != CB_DT_FLOAT32 && K > 0 && K % 8 == 0 && N % 8 == 0 && aligned(x, 16) &&
                       aligned(weight, 16) && K * N * 2 < (1LL << 31) && 128 * K * 2 < (1LL << 31);
     if (mfma) {
-        if (gmm_lds_enabled() && 256 * K * 2 < (1LL << 31) && 256 * N * 2 < (1LL << 31)) {
-            build_group_table(a.gt, group_list, E, GL_BM);
-            a.ntiles = (int)((N + GL_BN - 1) / GL_BN);
-            const int64_t blocks = (int64_t)a.gt.total_mtiles * a.ntiles;
-            if (blocks <= 0) return CB_OK;
-            const bool bf = x_dtype == CB_DT_BFLOAT16;
-            const void* kern = bf ? (a.trans ? (const void*)gmm_lds_kernel<true, true> : (const void*)gmm_lds_kernel<true, false>)
-                                  : (a.trans ? (const void*)gmm_lds_kernel<false, true> : (const void*)gmm_lds_kernel<false, false>);
-            set_dynamic_lds_once(kern, 2 * GL_STAGE);
-            if (bf && a.trans) hipLaunchKernelGGL((gmm_lds_kernel<true, true>), dim3((unsigned)blocks), dim3(GL_NT), 2 * GL_STAGE, st, a);
-            else if (bf) hipLaunchKernelGGL((gmm_lds_kernel<true, false>), dim3((unsigned)blocks), dim3(GL_NT), 2 * GL_STAGE, st, a);
-            else if (a.trans) hipLaunchKernelGGL((gmm_lds_kernel<false, true>), dim3((unsigned)blocks), dim3(GL_NT), 2 * GL_STAGE, st, a);
-            else hipLaunchKernelGGL((gmm_lds_kernel<false, false>), dim3((unsigned)blocks), dim3(GL_NT), 2 * GL_STAGE, st, a);
-            return check_launch();
+        // a test override of 128 selects the 128 x 128 register-staged kernel for every shape (it is
+        // otherwise taken only where a 256-row block of x or y passes 2 GiB)
+        const int tile = g_overrides.gmm_tile;
+        int pick = -1;
+        if (tile != 128 && 256 * K * 2 < (1LL << 31) && 256 * N * 2 < (1LL << 31))
+            pick = tile >= 1 && tile <= 6 ? tile - 1 : pick_gmm(a, group_list, E);
+        switch (pick) {
+            case 0: launch_gmm_tile<GmmT0>(a, group_list, E, st); return check_launch();
+            case 1: launch_gmm_tile<GmmT1>(a, group_list, E, st); return check_launch();
+            case 2: launch_gmm_tile<GmmT2>(a, group_list, E, st); return check_launch();
+            case 3: launch_gmm_tile<GmmT3>(a, group_list, E, st); return check_launch();
+            case 4: launch_gmm_tile<GmmT4>(a, group_list, E, st); return check_launch();
+            case 5: launch_gmm_tile<GmmT5>(a, group_list, E, st); return check_launch();
+            default: break;
         }
         build_group_table(a.gt, group_list, E, 128);
         a.ntiles = (int)((N + 127) / 128);

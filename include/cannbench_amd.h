@@ -201,8 +201,9 @@ int cb_grouped_matmul_swiglu_quant_noalloc(const int8_t* x, const int8_t* weight
  *                        gives up and leaves its output to the fix-up launch (default 2^20, about
  *                        2 s); a small value exercises the fix-up path, a negative one makes every
  *                        wait give up at once (the fix-up launch then writes every tile).
- *   gmm_tile             1 to 5 force one tile of the tiled GEMM (32 x 64, 64 x 128, 64 x 256,
- *                        128 x 128, 128 x 256) where its shape conditions hold; 128 forces the
+ *   gmm_tile             1 to 6 force one tile of the tiled GEMM (32 x 64, 64 x 128, 64 x 256,
+ *                        128 x 128, 128 x 256; 256 x 256 for GroupedMatmul only) where its shape
+ *                        conditions hold; 128 forces the
  *                        128 x 128 register-staged GroupedMatmul kernel for every fp16/bf16 shape.
  */
 void cb_set_test_overrides(int persistent_grid, int exchange_spin_limit, int gmm_tile);

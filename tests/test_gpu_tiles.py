@@ -1,12 +1,16 @@
-"""GPU parity of the tiled GEMMs between the skinny and the 256 x 256 kernels (QuantMatmul and the
-int8 grouped down-projection), each tile forced in turn through the library's test override: row
+"""GPU parity of the tiled GEMMs (QuantMatmul, the int8 grouped down-projection and the 16-bit
+GroupedMatmul), each tile forced in turn through the library's test override: row
 counts around the 32-row fragments and the tile edges, partial column tiles (N off every tile
 width), K of one 16-byte chunk, below, at and past a stage and the ring's depth, ragged and empty
 groups, every dequant flag and a batch.  The int32 sums are exact and the dequant chain rounds in
-the oracle's order, so the bar is bit equality."""
+the oracle's order, so the bar is bit equality; GroupedMatmul meets the bar of its own parity tests
+(one output ulp plus 1e-6 of sum |x w|, the fp32 sum's bound) and is bit-identical for both weight
+layouts."""
 import numpy as np
 import pytest
 import torch
+
+import test_gpu_gmm as gmm
 
 pytestmark = pytest.mark.gpu
 
@@ -79,3 +83,17 @@ def test_tile_batched(cb, tile):
     acc = np.matmul(x1.astype(np.int64), x2.astype(np.int64)).astype(np.float32) + bias.astype(np.float32)
     ref = torch.from_numpy(acc * scale).to(torch.bfloat16)
     assert torch.equal(out.cpu(), ref)
+
+
+@pytest.mark.parametrize("t", [1, 2, 3, 4, 5, 6])  # as above, then 256 x 256
+@pytest.mark.parametrize("counts,K,N", [([1, 0, 33, 64], 8, 24), ([127, 130, 2], 200, 264), ([257, 0, 31], 1032, 72)])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_tile_grouped_matmul(cb, orc, overrides, t, counts, K, N, dtype):
+    overrides(gmm_tile=t)
+    x, w, b, ends = gmm._inputs(counts, K, N, dtype, False, "f32", K + N)
+    args = dict(bias=b.to(DEV), split_item=2)
+    y = cb.grouped_matmul(x.to(DEV), w.to(DEV), ends, **args)[0]
+    yt = cb.grouped_matmul(x.to(DEV), w.transpose(1, 2).contiguous().to(DEV), ends, transpose_weight=True, **args)[0]
+    assert torch.equal(y.view(torch.int16), yt.view(torch.int16))
+    ref = orc.grouped_matmul(gmm.host(x, dtype), gmm.host(w, dtype), ends, b.numpy(), dtype=dtype, bias_dtype="f32")
+    gmm._check(y, ref, dtype, x.float(), w.float(), ends, False)
