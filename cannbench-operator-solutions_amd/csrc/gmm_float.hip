@@ -305,8 +305,8 @@ template <class OP, bool BT> using GmmT3 = TileCfg<OP, BT, 2, 4, 2, 1, 4, 1, 4, 
 template <class OP, bool BT> using GmmT4 = TileCfg<OP, BT, 2, 4, 2, 2, 2, 2, 3, 1>;  // 128 x 256, 8 waves
 template <class OP, bool BT> using GmmT5 = TileCfg<OP, BT, 2, 4, 4, 2, 1, 2, 4, 1>;  // 256 x 256, 8 waves
 
-// Estimated time of each tile over the call, in the terms of the int8 rule (moe_ops.hip: us per 128
-// bytes of K for a tile alone and in a full round of 256, us per round), combined with the bytes at
+// Estimated time of each tile over the call, in the terms of the int8 rule (tile_rounds_us, units of 128
+// bytes of K), combined with the bytes at
 // bw TB/s; the least is taken.  The choice does not look at the weight layout, so that [K][N] and
 // [N][K] storage of the same weights are summed in the same order and agree bit for bit.  Measured
 // us, 64 experts of 4096 x 4096 bf16, [K][N] / [N][K] weights (first: the 256 x 256 double-buffered
@@ -346,9 +346,7 @@ static int pick_gmm(const GmmFArgs& a, const int64_t* gl, int64_t E)
         const GmmCand& c = kGmmCand[i];
         const int64_t tiles = mt[c.bm == 32 ? 0 : c.bm == 64 ? 1 : c.bm == 128 ? 2 : 3] * ((a.N + c.bn - 1) / c.bn);
         if (tiles > (1 << 30)) continue;
-        const double rounds = (double)((tiles + 255) / 256);
-        const double full = rounds * (units * c.r + c.o), alone = units * c.p + c.o;
-        const double run = tiles >= 256 || full < alone ? full : alone + (full - alone) * (double)tiles / 256;
+        const double run = tile_rounds_us(tiles, units, c.p, c.r, c.o);
         const double mem = bytes / (c.bw * 1e6);
         const double t = run * run * run * run + mem * mem * mem * mem;
         if (best < 0 || t < best_t) {

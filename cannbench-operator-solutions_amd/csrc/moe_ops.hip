@@ -118,10 +118,10 @@ static int xcd_split(int ntiles, int64_t E, int64_t tile_row_bytes)
 }
 
 // ---- the dequant GEMM's choice of kernel -------------------------------------------------------
-// Estimated time in us of a BM x BN tile kernel over the call.  A tile alone on its CU takes p us per
-// 128 of K; with a tile on every CU, a round of 256 tiles takes r us per 128 of K plus o us (prologue
-// and epilogue); the bytes the call must move pass at bw TB/s, partly hidden by the multiplications
-// (the two times combine as the root of their squares); f us per call.  The constants are fitted to
+// Estimated time in us of a BM x BN tile kernel over the call (tile_rounds_us: p us per 128 of K for a
+// tile alone on its CU, r in a full round of 256, o per tile); the bytes the call must move pass at
+// bw TB/s, partly hidden by the multiplications (the two times combine as the root of their
+// squares); f us per call.  The constants are fitted to
 // the measured times below; the 256 x 256 ring core and the skinny kernel (at most 32 rows per
 // group) are candidates like the others, so the rule compares like with like.
 //   us, by rows (dense 7168 x 4096)          us, by rows per expert (256 x 2048 x 7168)
@@ -131,18 +131,19 @@ static int xcd_split(int ntiles, int64_t E, int64_t tile_row_bytes)
 //   64 x 256      36     36     41    75   140       680   736   801   988  1764
 //   128 x 128     26     27     35    69   134       921   956  1003  1065  2068
 //   128 x 256     40     42     45    61   118       797   841   907   999  1716
-//   ring          (40)   69     78    98   101       840   839   897   975  1404
+//   ring          (40)   69     78    98   101       840   800   830   930  1395
 //   skinny        55      -      -     -     -       624
 // With 2048 x 1024 weights 24 rows take 6.0 us (32 x 64) against 16.3 (skinny), 1024 rows 11.3
-// (64 x 128) against 28 (ring); 64 x 768 x 2048 with 200 rows per expert 45 (ring) against 63 (64 x 256).
+// (64 x 128) against 28 (ring); 64 x 768 x 2048 with 96 / 200 rows per expert 34 / 44 (ring) against
+// 41 / 63 (64 x 256).
 struct DeqCand {
     int bm, bn;
     double p, r, o, bw, f;
 };
 enum { DEQ_RING = 5, DEQ_SKINNY = 6 };
 static constexpr DeqCand kDeqCand[] = {
-    {32, 64, 0.30, 0.152, 1.5, 5.2, 2.0},   {64, 128, 0.36, 0.31, 2.7, 6.8, 2.0},  {64, 256, 0.58, 0.54, 4.2, 6.55, 2.0},
-    {128, 128, 0.42, 0.486, 6.8, 8.0, 2.0}, {128, 256, 0.64, 0.87, 10.0, 8.0, 2.0}, {256, 256, 1.55, 1.55, 10.0, 12.0, 2.0},
+    {32, 64, 0.30, 0.152, 1.5, 5.2, 2.0},   {64, 128, 0.36, 0.31, 2.7, 6.8, 2.0},  {64, 256, 0.58, 0.54, 4.6, 6.55, 2.0},
+    {128, 128, 0.34, 0.486, 6.8, 6.5, 2.0}, {128, 256, 0.55, 0.87, 10.6, 6.5, 2.0}, {256, 256, 1.55, 1.55, 12.0, 12.0, 2.0},
     {32, 256, 0.85, 0.30, 1.0, 6.3, 3.0},
 };
 
@@ -165,9 +166,9 @@ static int pick_deq(const GemmArgs& a, const int64_t* gl, int64_t E, int64_t bat
         if (i == DEQ_RING && !ring_ok) continue;
         const int64_t tiles = mt[c.bm == 32 ? 0 : c.bm == 64 ? 1 : c.bm == 128 ? 2 : 3] * ((a.N + c.bn - 1) / c.bn) * batch;
         if (tiles > (1 << 24) && best >= 0) continue;
-        const double rounds = (double)((tiles + 255) / 256);
-        const double full = rounds * (units * c.r + c.o);
-        const double run = full > units * c.p ? full : units * c.p;
+        // the ring core's epilogue leaves out 32-row fragments without valid rows
+        const double o = i == DEQ_RING ? 2.0 + 10.0 * (double)mt[0] / (8.0 * (double)mt[3]) : c.o;
+        const double run = tile_rounds_us(tiles, units, c.p, c.r, o);
         const double mem = bytes / (c.bw * 1e6);
         const double t = c.f + std::sqrt(run * run + mem * mem);
         if (best < 0 || t < best_t) {
