@@ -18,6 +18,8 @@
 
 namespace cb {
 
+constexpr int kDecRB = 2;  // 16-row blocks per tile (3: 48 rows, level with the prefill kernel; 4 spills)
+
 // The product, SwiGLU and row maxima of one tile: RB 16-row blocks of expert g from row r0 on (rows
 // below r1) x 128 act columns.  Lane (q, c), c < 8, ends with act[rb][j] = act of row r0 + 16 rb +
 // 4 q + wave, act column 128 ct + 16 c + j, and rmax[rb] = the row's maximum |act| over the tile (in
@@ -26,10 +28,10 @@ namespace cb {
 // the weight stream, and a second pass for rows 17 to 32 doubled it (7168 x 4096 x 256 experts with
 // 16 rows each on average, 28 at most: 1.55 ms, 1.18 ms in one pass; 2048 rows, 16 at most: 1.16 ms
 // either way).
-template <int RB, int RBM>
+template <int RB>
 __device__ __forceinline__ void decode_tile_act_n(const GemmArgs& a, const int g, const int ct, const int r0,
-                                                  const int r1, int (&red)[3][4][16][64], float (&act)[RBM][16],
-                                                  u32 (&rmax)[RBM])
+                                                  const int r1, int (&red)[3][4][16][64], float (&act)[kDecRB][16],
+                                                  u32 (&rmax)[kDecRB])
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int q = lane >> 4, c = lane & 15;
@@ -66,7 +68,7 @@ __device__ __forceinline__ void decode_tile_act_n(const GemmArgs& a, const int g
         skinny_load_chunk(xres, wres, lane_off, (uint32_t)N, q, kc + 12, R1, A1);
     }
 #pragma unroll
-    for (int rb = 0; rb < RBM; ++rb) {
+    for (int rb = 0; rb < kDecRB; ++rb) {
         rmax[rb] = 0u;
 #pragma unroll
         for (int j = 0; j < 16; ++j) act[rb][j] = 0.0f;
@@ -99,27 +101,24 @@ __device__ __forceinline__ void decode_tile_act_n(const GemmArgs& a, const int g
 }
 
 // The smallest variant that holds the tile's rows.
-template <int RBM>
 __device__ __forceinline__ void decode_tile_act(const GemmArgs& a, const int g, const int ct, const int r0, const int r1,
-                                                int (&red)[3][4][16][64], float (&act)[RBM][16], u32 (&rmax)[RBM])
+                                                int (&red)[3][4][16][64], float (&act)[kDecRB][16], u32 (&rmax)[kDecRB])
 {
     if (r1 - r0 <= 16) decode_tile_act_n<1>(a, g, ct, r0, r1, red, act, rmax);
-    else if (RBM == 2 || r1 - r0 <= 32) decode_tile_act_n<2>(a, g, ct, r0, r1, red, act, rmax);
-    else if constexpr (RBM > 2) decode_tile_act_n<RBM>(a, g, ct, r0, r1, red, act, rmax);
+    else decode_tile_act_n<2>(a, g, ct, r0, r1, red, act, rmax);
 }
 
 // Row maxima exchange through self-validating slots: tile (g, ct) stores, for each of its rows r,
 // slot[r * ntiles + ct] = |act| maximum bits | 0x80000000 (the bit marks the slot as written; the
 // workspace starts zeroed).  A row's final maximum is the maximum over its ntiles slots once every
 // slot carries the mark, so no separate arrival count (and no wait for the stores) is needed.
-template <int RBM>
 __device__ __forceinline__ void decode_publish(const GemmArgs& a, const int ct, const int r0, const int r1,
-                                               const u32 (&rmax)[RBM])
+                                               const u32 (&rmax)[kDecRB])
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int q = lane >> 4, c = lane & 15;
 #pragma unroll
-    for (int rb = 0; rb < RBM; ++rb) {
+    for (int rb = 0; rb < kDecRB; ++rb) {
         const int row = r0 + 16 * rb + 4 * q + wave;
         if (c == 0 && row < r1)
             __hip_atomic_store(a.epi.amax + (int64_t)row * a.ntiles + ct, rmax[rb] | 0x80000000u, __ATOMIC_RELAXED,
@@ -129,8 +128,7 @@ __device__ __forceinline__ void decode_publish(const GemmArgs& a, const int ct, 
 
 // The final row maxima of this lane's rows (every lane of a 16-lane group gets its row's value),
 // polling until all ntiles slots are marked, at most spin_limit times.  Returns false on timeout.
-template <int RBM>
-__device__ __forceinline__ bool decode_gather(const GemmArgs& a, const int r0, const int r1, float (&am)[RBM])
+__device__ __forceinline__ bool decode_gather(const GemmArgs& a, const int r0, const int r1, float (&am)[kDecRB])
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int q = lane >> 4, c = lane & 15;
@@ -138,7 +136,7 @@ __device__ __forceinline__ bool decode_gather(const GemmArgs& a, const int r0, c
     for (int spins = 0;; ++spins) {
         bool all = true;
 #pragma unroll
-        for (int rb = 0; rb < RBM; ++rb) {
+        for (int rb = 0; rb < kDecRB; ++rb) {
             const int row = r0 + 16 * rb + 4 * q + wave;
             u32 m = 0u, ok = 1u;
             if (r0 + 16 * rb < r1 && row < r1) {
@@ -171,9 +169,8 @@ __device__ __forceinline__ bool decode_gather(const GemmArgs& a, const int r0, c
 
 // y = rint16(act * 127 / amax) with amax floored at FLT_MIN (an all-zero row gives 0 * inf = NaN
 // -> 0), 16 bytes per lane; column tile 0 writes y_scale.
-template <int RBM>
 __device__ __forceinline__ void decode_tile_quant(const GemmArgs& a, const int ct, const int r0, const int r1,
-                                                  const float (&act)[RBM][16], const float (&amax)[RBM])
+                                                  const float (&act)[kDecRB][16], const float (&amax)[kDecRB])
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int q = lane >> 4, c = lane & 15;
@@ -181,7 +178,7 @@ __device__ __forceinline__ void decode_tile_quant(const GemmArgs& a, const int c
     const int64_t H = e.H;
     const int64_t ocol = (int64_t)ct * 128 + 16 * (c & 7);
 #pragma unroll
-    for (int rb = 0; rb < RBM; ++rb) {
+    for (int rb = 0; rb < kDecRB; ++rb) {
         const int row = r0 + 16 * rb + 4 * q + wave;
         if (row < r1) {
             float am = amax[rb];
@@ -215,11 +212,10 @@ __device__ __forceinline__ void decode_tile_quant(const GemmArgs& a, const int c
 // for the fix-up launch (which redoes the whole tile) and stores nothing.  no_wait: the tile is
 // left to the fix-up launch without waiting (status bit 1 instead of the timeout bit 0, so the
 // other waits of the call still wait).
-template <int RBM>
 __device__ __forceinline__ void decode_finish(const GemmArgs& a, const int mt, const int ct, const int r0, const int r1,
-                                              const float (&act)[RBM][16], const bool no_wait = false)
+                                              const float (&act)[kDecRB][16], const bool no_wait = false)
 {
-    float am[RBM];
+    float am[kDecRB];
     // a negative poll limit (test hook) gives up at once
     if (!no_wait && a.epi.spin_limit >= 0 && decode_gather(a, r0, r1, am)) {
         decode_tile_quant(a, ct, r0, r1, act, am);
@@ -246,11 +242,10 @@ __device__ __forceinline__ void decode_finish(const GemmArgs& a, const int mt, c
 // workgroup whose own D lies in its own P's expert (possible only with few workgroups, e.g. a
 // partly resident grid).  Such a workgroup does not wait: it leaves P to the fix-up launch and
 // goes on to D, so the waits cannot form a cycle.
-template <int RBM>
 __global__ __launch_bounds__(256, 1) void gmsq_decode_kernel(const GemmArgs a)
 {
     __shared__ int red[3][4][16][64];      // partial sums handed to the wave that owns them (48 KiB)
-    __shared__ float park[4][4][8][RBM][16];  // the deferred tile's activations (lanes c < 8; 8 KiB per row block)
+    __shared__ float park[4][4][8][kDecRB][16];  // the deferred tile's activations (lanes c < 8; 8 KiB per row block)
     __shared__ u32 next_t, pend_t;
     const int ntl = a.ntiles;
     const int count = a.gt.total_mtiles * ntl;
@@ -269,11 +264,11 @@ __global__ __launch_bounds__(256, 1) void gmsq_decode_kernel(const GemmArgs a)
         if (threadIdx.x == 0) nt_pending = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const int mt = t / ntl, ct = t % ntl;
         const int g = group_of_tile(a.gt, mt);
-        const int r0 = (g ? a.gt.row_end[g - 1] : 0) + (mt - a.gt.tile_start[g]) * 16 * RBM;
-        const int r1 = r0 + 16 * RBM < a.gt.row_end[g] ? r0 + 16 * RBM : a.gt.row_end[g];
+        const int r0 = (g ? a.gt.row_end[g - 1] : 0) + (mt - a.gt.tile_start[g]) * 16 * kDecRB;
+        const int r1 = r0 + 16 * kDecRB < a.gt.row_end[g] ? r0 + 16 * kDecRB : a.gt.row_end[g];
         {
-            float act[RBM][16];
-            u32 rmax[RBM];
+            float act[kDecRB][16];
+            u32 rmax[kDecRB];
             decode_tile_act(a, g, ct, r0, r1, red, act, rmax);
             decode_publish(a, ct, r0, r1, rmax);
             if (pm >= 0) {
@@ -283,16 +278,16 @@ __global__ __launch_bounds__(256, 1) void gmsq_decode_kernel(const GemmArgs a)
                 __syncthreads();
                 const int pend = (int)pend_t;
                 const bool self_dep = pend < count && pend / ntl == pm;
-                float pact[RBM][16];
+                float pact[kDecRB][16];
 #pragma unroll
-                for (int rb = 0; rb < RBM; ++rb)
+                for (int rb = 0; rb < kDecRB; ++rb)
 #pragma unroll
                     for (int j = 0; j < 16; ++j) pact[rb][j] = c < 8 ? park[wave][q][c & 7][rb][j] : 0.0f;
                 decode_finish(a, pm, pct, pr0, pr1, pact, self_dep);
             }
             if (c < 8) {
 #pragma unroll
-                for (int rb = 0; rb < RBM; ++rb)
+                for (int rb = 0; rb < kDecRB; ++rb)
 #pragma unroll
                     for (int j = 0; j < 16; ++j) park[wave][q][c][rb][j] = act[rb][j];
             }
@@ -307,9 +302,9 @@ __global__ __launch_bounds__(256, 1) void gmsq_decode_kernel(const GemmArgs a)
         __syncthreads();  // next_t is rewritten by the next draw
     }
     if (pm >= 0) {
-        float pact[RBM][16];
+        float pact[kDecRB][16];
 #pragma unroll
-        for (int rb = 0; rb < RBM; ++rb)
+        for (int rb = 0; rb < kDecRB; ++rb)
 #pragma unroll
             for (int j = 0; j < 16; ++j) pact[rb][j] = c < 8 ? park[wave][q][c & 7][rb][j] : 0.0f;
         decode_finish(a, pm, pct, pr0, pr1, pact);
@@ -317,7 +312,6 @@ __global__ __launch_bounds__(256, 1) void gmsq_decode_kernel(const GemmArgs a)
 }
 
 // Fix-up launch: tiles marked in redo[mt * ntiles + ct], recomputed with the final row maxima.
-template <int RBM>
 __global__ __launch_bounds__(256, 1) void gmsq_decode_fixup_kernel(const GemmArgs a)
 {
     __shared__ int red[3][4][16][64];
@@ -330,12 +324,12 @@ __global__ __launch_bounds__(256, 1) void gmsq_decode_fixup_kernel(const GemmArg
             continue;
         const int mt = t / a.ntiles, ct = t % a.ntiles;
         const int g = group_of_tile(a.gt, mt);
-        const int r0 = (g ? a.gt.row_end[g - 1] : 0) + (mt - a.gt.tile_start[g]) * 16 * RBM;
-        const int r1 = r0 + 16 * RBM < a.gt.row_end[g] ? r0 + 16 * RBM : a.gt.row_end[g];
-        float act[RBM][16];
-        u32 rmax[RBM];
+        const int r0 = (g ? a.gt.row_end[g - 1] : 0) + (mt - a.gt.tile_start[g]) * 16 * kDecRB;
+        const int r1 = r0 + 16 * kDecRB < a.gt.row_end[g] ? r0 + 16 * kDecRB : a.gt.row_end[g];
+        float act[kDecRB][16];
+        u32 rmax[kDecRB];
         decode_tile_act(a, g, ct, r0, r1, red, act, rmax);
-        float am[RBM];
+        float am[kDecRB];
         (void)decode_gather(a, r0, r1, am);  // every slot was written before this launch
         decode_tile_quant(a, ct, r0, r1, act, am);
         __syncthreads();

@@ -305,17 +305,17 @@ extern "C" int64_t cb_grouped_matmul_swiglu_quant_workspace_size(int64_t M, int6
 }
 
 // GroupedMatmulSwigluQuant by weight streaming with the requant fused (per-expert exchange; y at any
-// alignment), row tiles of 16 RBM rows, on a persistent grid of one workgroup per CU (each wave keeps
+// alignment), row tiles of 16 kDecRB rows, on a persistent grid of one workgroup per CU (each wave keeps
 // two weight chunks in flight in its registers) drawing tiles from one ticket in expert order.
 // Returns -1 when the kernel cannot be resident.
-template <int RBM, class Clear>
+template <class Clear>
 static int launch_gmsq_decode(GemmArgs& a, const int64_t* group_list, int64_t E, int ntl, Clear&& clear_ws, hipStream_t st)
 {
     const int cus = device_cus();
     int resident = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, (const void*)gmsq_decode_kernel<RBM>, 256, 0) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, (const void*)gmsq_decode_kernel, 256, 0) != hipSuccess)
         resident = 0;
-    build_group_table(a.gt, group_list, E, 16 * RBM);
+    build_group_table(a.gt, group_list, E, 16 * kDecRB);
     const int64_t tiles = (int64_t)a.gt.total_mtiles * ntl;
     int grid = (resident < 1 ? resident : 1) * cus;
     if (g_overrides.persistent_grid > 0 && resident >= 1) grid = g_overrides.persistent_grid;  // test hook
@@ -325,9 +325,9 @@ static int launch_gmsq_decode(GemmArgs& a, const int64_t* group_list, int64_t E,
     clear_ws(tiles);
     {
         TimedLaunch timed(st);
-        hipLaunchKernelGGL(gmsq_decode_kernel<RBM>, dim3((unsigned)grid), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(gmsq_decode_kernel, dim3((unsigned)grid), dim3(256), 0, st, a);
     }
-    hipLaunchKernelGGL(gmsq_decode_fixup_kernel<RBM>, dim3((unsigned)(tiles < 512 ? tiles : 512)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(gmsq_decode_fixup_kernel, dim3((unsigned)(tiles < 512 ? tiles : 512)), dim3(256), 0, st, a);
     return check_launch();
 }
 
@@ -421,7 +421,7 @@ static int gmsq_impl(const int8_t* x, int64_t x_rows, const int32_t* row_index, 
     }
     if (fused && fast && a.gt.max_rows <= kSkinnyMaxRows) {
         // decode-shaped groups
-        const int rc = launch_gmsq_decode<2>(a, group_list, E, ntl, clear_ws, st);
+        const int rc = launch_gmsq_decode(a, group_list, E, ntl, clear_ws, st);
         if (rc >= 0) return rc;
     }
     // any other shape or alignment: two passes over the products (row maxima, then the requant)
