@@ -6,8 +6,8 @@
 //
 // 16-bit inputs run on v_mfma_f32_32x32x16_{f16,bf16} through the tiles of gemm_tile.hpp (32 x 64 to
 // 256 x 256, chosen by pick_gmm), fp32 accumulation, the bias added in fp32, one
-// round-to-nearest-even narrowing.  Rows or outputs past 32-bit offsets take a 128 x 128
-// register-staged kernel.  fp32 inputs and shapes off the vector path
+// round-to-nearest-even narrowing.  Rows or outputs past 32-bit offsets and outputs off 16-byte
+// alignment take a 128 x 128 register-staged kernel.  fp32 inputs and shapes off the vector path
 // (K or N not a multiple of 8, misaligned operands, 32-bit offsets exceeded) take a plain fp32 loop.
 #include <cstdlib>
 #include <cstring>
@@ -399,10 +399,11 @@ extern "C" int cb_grouped_matmul(const void* x, const void* weight, const void* 
                       aligned(weight, 16) && K * N * 2 < (1LL << 31) && 128 * K * 2 < (1LL << 31);
     if (mfma) {
         // a test override of 128 selects the 128 x 128 register-staged kernel for every shape (it is
-        // otherwise taken only where a 256-row block of x or y passes 2 GiB)
+        // otherwise taken only where a 256-row block of x or y passes 2 GiB or y is not 16-byte
+        // aligned: it stores single values)
         const int tile = g_overrides.gmm_tile;
         int pick = -1;
-        if (tile != 128 && 256 * K * 2 < (1LL << 31) && 256 * N * 2 < (1LL << 31))
+        if (tile != 128 && 256 * K * 2 < (1LL << 31) && 256 * N * 2 < (1LL << 31) && aligned(y, 16))  // 16-byte stores
             pick = tile >= 1 && tile <= 6 ? tile - 1 : pick_gmm(a, group_list, E);
         switch (pick) {
             case 0: launch_gmm_tile<GmmT0>(a, group_list, E, st); return check_launch();

@@ -97,3 +97,21 @@ def test_tile_grouped_matmul(cb, orc, overrides, t, counts, K, N, dtype):
     assert torch.equal(y.view(torch.int16), yt.view(torch.int16))
     ref = orc.grouped_matmul(gmm.host(x, dtype), gmm.host(w, dtype), ends, b.numpy(), dtype=dtype, bias_dtype="f32")
     gmm._check(y, ref, dtype, x.float(), w.float(), ends, False)
+
+
+@pytest.mark.parametrize("off", [1, 2, 4])  # elements: y at 2, 4 and 8 bytes past a 16-byte boundary
+def test_grouped_matmul_unaligned_output(cb, off):
+    """An output off 16-byte alignment (possible through the C ABI) takes the kernel with single-value
+    stores and leaves its neighbours alone."""
+    x, w, b, ends = gmm._inputs([70, 3], 64, 40, "bf16", False, "f32", 5)
+    xd, wd, bd = x.to(DEV), w.to(DEV), b.to(DEV)
+    ref = cb.grouped_matmul(xd, wd, ends, bias=bd, split_item=2)[0]
+    buf = torch.full((73 * 40 + 16,), 7.0, dtype=torch.bfloat16, device=DEV)
+    rc = cb._lib.load().cb_grouped_matmul(
+        xd.data_ptr(), wd.data_ptr(), bd.data_ptr(), cb._lib.CB_DT_BFLOAT16, cb._lib.CB_DT_FLOAT32,
+        cb._lib.int64_array(ends), 2, 73, 64, 40, 2, 0, buf.data_ptr() + 2 * off, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    got = buf[off:off + 73 * 40].view(73, 40).float()
+    # the two kernels sum in different orders: at most one bf16 step apart
+    assert ((got - ref.float()).abs() <= ref.float().abs() * 2.0 ** -7 + 1e-5).all()
+    assert (buf[:off] == 7).all() and (buf[off + 73 * 40:] == 7).all()
