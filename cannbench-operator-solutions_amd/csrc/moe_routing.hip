@@ -1021,13 +1021,7 @@ extern "C" int cb_dequant_swiglu_quant(const void* x, int x_dtype, int64_t M, in
         int threads = (int)(((nvh + NVmax - 1) / NVmax + 63) / 64 * 64);
         threads = threads < 64 ? 64 : threads;
         const int64_t passes = (nvh + threads - 1) / threads;
-        // two rows per workgroup (the second row's loads in flight while the first is reduced), and at
-        // least enough workgroups to fill every CU twice.  Longer walks drift apart: 131072 x 4096
-        // int32 takes 413 us with 2 rows each, 424 with 4, 530 with 16, 468 with 64, and 452 with 1;
-        // bf16 211, 231, 239, 251 and 226; 16384 rows int32 53.8 against 58.7 with 8
-        const int64_t per_cu = 2048 / threads;  // waves resident per CU at this block size (occupancy 8)
-        const int64_t fill = 256 * per_cu * 2, half = (M + 1) / 2;
-        const int64_t nblk = M < fill ? M : (half > fill ? half : fill);
+        const int64_t nblk = dqsq_blocks(M, threads);
         const dim3 pgrid((unsigned)nblk);
 #define CB_DQSQ_L(XDTV, NVV, QSV, LV)                                                              \
     hipLaunchKernelGGL((dqsq_vec_kernel<XDTV, NVV, QSV, LV>), pgrid, dim3(threads), 0, st, x, M, H,  \

@@ -161,6 +161,19 @@ def test_dequant_swiglu_quant(cb, orc, xdt, qs, left, M, H):
     _assert_i8(y.cpu().numpy(), ry, f"dqsq {xdt} M={M} H={H}")
 
 
+def test_dequant_swiglu_quant_rows_past_the_dispatch_limit(cb):
+    """2^27 + 5 rows of 16 columns, 64 threads each: half as many workgroups are one too many for a
+    dispatch (32 bits of work-items), so the workgroups walk more rows.  Every row is computed by
+    itself: slices equal calls on those rows alone, bit for bit."""
+    M = (1 << 27) + 5
+    x = torch.empty((M, 16), dtype=torch.bfloat16, device=DEV)
+    x.normal_(generator=torch.Generator(device=DEV).manual_seed(1))
+    y, s = cb.dequant_swiglu_quant(x)
+    for a, b in ((0, 3000), ((1 << 26) - 100, (1 << 26) + 100), (M - 3000, M)):
+        yr, sr = cb.dequant_swiglu_quant(x[a:b].clone())
+        assert torch.equal(y[a:b], yr) and torch.equal(s[a:b], sr)
+
+
 def test_dequant_swiglu_quant_zero_rows_and_checks(cb):
     x = torch.zeros(3, 64, dtype=torch.bfloat16, device=DEV)
     y, s = cb.dequant_swiglu_quant(x)
