@@ -305,58 +305,6 @@ template <class OP, bool BT> using GmmT3 = TileCfg<OP, BT, 2, 4, 2, 1, 4, 1, 4, 
 template <class OP, bool BT> using GmmT4 = TileCfg<OP, BT, 2, 4, 2, 2, 2, 2, 3, 1>;  // 128 x 256, 8 waves
 template <class OP, bool BT> using GmmT5 = TileCfg<OP, BT, 2, 4, 4, 2, 1, 2, 4, 1>;  // 256 x 256, 8 waves
 
-// Estimated time of each tile over the call, in the terms of the int8 rule (tile_rounds_us, units of 128
-// bytes of K), combined with the bytes at
-// bw TB/s; the least is taken.  The choice does not look at the weight layout, so that [K][N] and
-// [N][K] storage of the same weights are summed in the same order and agree bit for bit.  Measured
-// us, 64 experts of 4096 x 4096 bf16, [K][N] / [N][K] weights (first: the 256 x 256 double-buffered
-// kernel these replace):
-//   rows per expert     8          24         64         128        256         512
-//   (replaced)       479 / 510  484 / 527  514 / 538  544 / 566  871 / 862  1377 / 1352
-//   32 x 64          377 / 362  419 / 389  583 / 575  855 / 866    -           -
-//   64 x 128         374 / 363  388 / 372  467 / 443  601 / 605  936 / 946     -
-//   64 x 256         346 / 375  354 / 388  444 / 494  540 / 635  870 / 1017    -
-//   128 x 128        402 / 384  409 / 395  437 / 414  554 / 549  845 / 837  1430 / 1401
-//   128 x 256        355 / 372     -       384 / 394  495 / 490  750 / 764  1234 / 1226
-//   256 x 256        409 / 425     -       457 / 485  487 / 544  801 / 875  1241 / 1323
-// 8 experts of 2048 x 1536, 8 rows each: 53 -> 13.6 (32 x 64); 1024 rows each: 69 -> 62 (256 x 256).
-struct GmmCand {
-    int bm, bn;
-    double p, r, o, bw;
-};
-static constexpr GmmCand kGmmCand[] = {
-    {32, 64, 0.30, 0.152, 1.5, 6.0},  {64, 128, 0.36, 0.34, 2.7, 6.0}, {64, 256, 0.58, 0.66, 5.0, 6.2},
-    {128, 128, 0.42, 0.51, 6.8, 6.2}, {128, 256, 0.90, 0.92, 9.0, 6.2}, {256, 256, 1.30, 1.75, 8.0, 6.2},
-};
-
-static int pick_gmm(const GmmFArgs& a, const int64_t* gl, int64_t E)
-{
-    const double units = (double)((a.K + 63) / 64);
-    int64_t mt[4] = {0, 0, 0, 0}, used = 0, prev = 0;  // row tiles of 32, 64, 128 and 256 rows
-    for (int64_t g = 0; g < E; ++g) {
-        const int64_t rows = gl[g] - prev;
-        for (int j = 0; j < 4; ++j) mt[j] += (rows + (32 << j) - 1) >> (5 + j);
-        used += rows > 0;
-        prev = gl[g];
-    }
-    const double bytes = 2.0 * ((double)used * a.K * a.N + (double)a.M * (a.K + a.N));
-    double best_t = 0;
-    int best = -1;
-    for (int i = 0; i < (int)(sizeof(kGmmCand) / sizeof(kGmmCand[0])); ++i) {
-        const GmmCand& c = kGmmCand[i];
-        const int64_t tiles = mt[c.bm == 32 ? 0 : c.bm == 64 ? 1 : c.bm == 128 ? 2 : 3] * ((a.N + c.bn - 1) / c.bn);
-        if (tiles > (1 << 30)) continue;
-        const double run = tile_rounds_us(tiles, units, c.p, c.r, c.o);
-        const double mem = bytes / (c.bw * 1e6);
-        const double t = run * run * run * run + mem * mem * mem * mem;
-        if (best < 0 || t < best_t) {
-            best = i;
-            best_t = t;
-        }
-    }
-    return best;
-}
-
 }  // namespace cb
 
 using namespace cb;
@@ -404,7 +352,7 @@ extern "C" int cb_grouped_matmul(const void* x, const void* weight, const void* 
         const int tile = g_overrides.gmm_tile;
         int pick = -1;
         if (tile != 128 && 256 * K * 2 < (1LL << 31) && 256 * N * 2 < (1LL << 31) && aligned(y, 16))  // 16-byte stores
-            pick = tile >= 1 && tile <= 6 ? tile - 1 : pick_gmm(a, group_list, E);
+            pick = tile >= 1 && tile <= 6 ? tile - 1 : pick_gmm(group_list, E, M, K, N);
         switch (pick) {
             case 0: launch_gmm_tile<GmmT0>(a, group_list, E, st); return check_launch();
             case 1: launch_gmm_tile<GmmT1>(a, group_list, E, st); return check_launch();

@@ -69,18 +69,6 @@ inline void build_group_table(GroupTable& t, const int64_t* gl, int64_t E, int b
     t.max_rows = mx;
 }
 
-// Time model of a tiled GEMM for the rules that choose a tile: a tile alone on its CU takes p us per
-// K unit and o us for its prologue and epilogue; with a tile on each of the 256 CUs a round takes r us
-// per K unit and o us (r above p: the CUs share L2 and fabric bandwidth; below: several workgroups
-// per CU hide each other's latency).
-inline double tile_rounds_us(int64_t tiles, double units, double p, double r, double o)
-{
-    const double alone = units * p + o, full = units * r + o;
-    if (tiles < 256 && full > alone) return alone + (full - alone) * (double)tiles / 256;
-    const double t = (double)((tiles + 255) / 256) * full;
-    return t > alone ? t : alone;
-}
-
 inline int check_launch()
 {
     return hipGetLastError() == hipSuccess ? CB_OK : CB_ERR_LAUNCH;

@@ -2,6 +2,7 @@
 // that a host program can check them at sizes no test allocates (tests/launch_rules).
 #pragma once
 
+#include <cmath>
 #include <stdint.h>
 
 namespace cb {
@@ -23,6 +24,140 @@ inline int64_t dqsq_blocks(int64_t M, int64_t threads)
     const int64_t fill = 256 * per_cu * 2, half = (M + 1) / 2;
     const int64_t want = M < fill ? M : (half > fill ? half : fill), most = ((1LL << 32) - 1) / threads;
     return want < most ? want : most;
+}
+
+// Time model of a tiled GEMM for the rules that choose a tile: a tile alone on its CU takes p us per
+// K unit and o us for its prologue and epilogue; with a tile on each of the 256 CUs a round takes r us
+// per K unit and o us (r above p: the CUs share L2 and fabric bandwidth; below: several workgroups
+// per CU hide each other's latency).
+inline double tile_rounds_us(int64_t tiles, double units, double p, double r, double o)
+{
+    const double alone = units * p + o, full = units * r + o;
+    if (tiles < 256 && full > alone) return alone + (full - alone) * (double)tiles / 256;
+    const double t = (double)((tiles + 255) / 256) * full;
+    return t > alone ? t : alone;
+}
+
+// ---- the dequant GEMM's choice of kernel (QuantMatmul, the grouped down-projection) -------------
+// Estimated time in us of a BM x BN tile kernel over the call (tile_rounds_us: p us per 128 of K for a
+// tile alone on its CU, r in a full round of 256, o per tile); the bytes the call must move pass at
+// bw TB/s, partly hidden by the multiplications (the two times combine as the root of their
+// squares); f us per call.  The constants are fitted to
+// the measured times below; the 256 x 256 ring core and the skinny kernel (at most 32 rows per
+// group) are candidates like the others, so the rule compares like with like.
+//   us, by rows (dense 7168 x 4096)          us, by rows per expert (256 x 2048 x 7168)
+//                  24    300   1024  2048  4096       8     24    47    96    256
+//   32 x 64       18.3   38     87   165   321       836   912  1257  1971  4750
+//   64 x 128      23.2   24     44    84   161       705   782   829  1054  2019
+//   64 x 256      36     36     41    75   140       680   736   801   988  1764
+//   128 x 128     26     27     35    69   134       921   956  1003  1065  2068
+//   128 x 256     40     42     45    61   118       797   841   907   999  1716
+//   ring          (40)   69     78    98   101       840   800   830   930  1395
+//   skinny        55      -      -     -     -       624
+// With 2048 x 1024 weights 24 rows take 6.0 us (32 x 64) against 16.3 (skinny), 1024 rows 11.3
+// (64 x 128) against 28 (ring); 64 x 768 x 2048 with 96 / 200 rows per expert 34 / 44 (ring) against
+// 41 / 63 (64 x 256).
+inline constexpr int kSkinnyMaxRows = 32;  // groups up to this many rows can take the skinny core
+
+struct DeqCand {
+    int bm, bn, threads;  // threads 0: the launch does not grow with the number of tiles
+    double p, r, o, bw, f;
+};
+enum { DEQ_RING = 5, DEQ_SKINNY = 6 };
+inline constexpr DeqCand kDeqCand[] = {
+    {32, 64, 256, 0.30, 0.152, 1.5, 5.2, 2.0},   {64, 128, 256, 0.36, 0.31, 2.7, 6.8, 2.0},
+    {64, 256, 256, 0.58, 0.54, 4.6, 6.55, 2.0},  {128, 128, 512, 0.34, 0.486, 6.8, 6.5, 2.0},
+    {128, 256, 512, 0.55, 0.87, 10.6, 6.5, 2.0}, {256, 256, 0, 1.55, 1.55, 12.0, 12.0, 2.0},
+    {32, 256, 0, 0.85, 0.30, 1.0, 6.3, 3.0},
+};
+
+// The index of the cheapest candidate, -1 where none fits a dispatch.
+inline int pick_deq(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N, int64_t batch, bool ring_ok)
+{
+    const double units = (double)((K + 127) / 128);
+    int64_t mt[4] = {0, 0, 0, 0}, used = 0, prev = 0, max_rows = 0;  // row tiles of 32, 64, 128 and 256 rows
+    for (int64_t g = 0; g < E; ++g) {
+        const int64_t rows = gl[g] - prev;
+        max_rows = rows > max_rows ? rows : max_rows;
+        for (int j = 0; j < 4; ++j) mt[j] += (rows + (32 << j) - 1) >> (5 + j);
+        used += rows > 0;
+        prev = gl[g];
+    }
+    const double bytes = (double)batch * ((double)used * K * N + (double)M * (K + 2 * N));
+    double best_t = 0;
+    int best = -1;
+    for (int i = 0; i < (int)(sizeof(kDeqCand) / sizeof(kDeqCand[0])); ++i) {
+        const DeqCand& c = kDeqCand[i];
+        if (i == DEQ_SKINNY && max_rows > kSkinnyMaxRows) continue;
+        if (i == DEQ_RING && !ring_ok) continue;
+        int64_t tiles = mt[c.bm == 32 ? 0 : c.bm == 64 ? 1 : c.bm == 128 ? 2 : 3] * ((N + c.bn - 1) / c.bn);
+        if (!grid_fits(tiles, c.threads)) continue;
+        tiles *= batch;
+        // the ring core's epilogue leaves out 32-row fragments without valid rows
+        const double o = i == DEQ_RING ? 2.0 + 10.0 * (double)mt[0] / (8.0 * (double)mt[3]) : c.o;
+        const double run = tile_rounds_us(tiles, units, c.p, c.r, o);
+        const double mem = bytes / (c.bw * 1e6);
+        const double t = c.f + std::sqrt(run * run + mem * mem);
+        if (best < 0 || t < best_t) {
+            best = i;
+            best_t = t;
+        }
+    }
+    return best;
+}
+
+// ---- the 16-bit GroupedMatmul's choice of tile --------------------------------------------------
+// Estimated time of each tile over the call, in the terms of the int8 rule (tile_rounds_us, units of 128
+// bytes of K), combined with the bytes at
+// bw TB/s; the least is taken.  The choice does not look at the weight layout, so that [K][N] and
+// [N][K] storage of the same weights are summed in the same order and agree bit for bit.  Measured
+// us, 64 experts of 4096 x 4096 bf16, [K][N] / [N][K] weights (first: the 256 x 256 double-buffered
+// kernel these replace):
+//   rows per expert     8          24         64         128        256         512
+//   (replaced)       479 / 510  484 / 527  514 / 538  544 / 566  871 / 862  1377 / 1352
+//   32 x 64          377 / 362  419 / 389  583 / 575  855 / 866    -           -
+//   64 x 128         374 / 363  388 / 372  467 / 443  601 / 605  936 / 946     -
+//   64 x 256         346 / 375  354 / 388  444 / 494  540 / 635  870 / 1017    -
+//   128 x 128        402 / 384  409 / 395  437 / 414  554 / 549  845 / 837  1430 / 1401
+//   128 x 256        355 / 372     -       384 / 394  495 / 490  750 / 764  1234 / 1226
+//   256 x 256        409 / 425     -       457 / 485  487 / 544  801 / 875  1241 / 1323
+// 8 experts of 2048 x 1536, 8 rows each: 53 -> 13.6 (32 x 64); 1024 rows each: 69 -> 62 (256 x 256).
+struct GmmCand {
+    int bm, bn, threads;
+    double p, r, o, bw;
+};
+inline constexpr GmmCand kGmmCand[] = {
+    {32, 64, 256, 0.30, 0.152, 1.5, 6.0},  {64, 128, 256, 0.36, 0.34, 2.7, 6.0}, {64, 256, 256, 0.58, 0.66, 5.0, 6.2},
+    {128, 128, 512, 0.42, 0.51, 6.8, 6.2}, {128, 256, 512, 0.90, 0.92, 9.0, 6.2}, {256, 256, 512, 1.30, 1.75, 8.0, 6.2},
+};
+
+// The index of the cheapest tile, -1 where none fits a dispatch.
+inline int pick_gmm(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N)
+{
+    const double units = (double)((K + 63) / 64);
+    int64_t mt[4] = {0, 0, 0, 0}, used = 0, prev = 0;  // row tiles of 32, 64, 128 and 256 rows
+    for (int64_t g = 0; g < E; ++g) {
+        const int64_t rows = gl[g] - prev;
+        for (int j = 0; j < 4; ++j) mt[j] += (rows + (32 << j) - 1) >> (5 + j);
+        used += rows > 0;
+        prev = gl[g];
+    }
+    const double bytes = 2.0 * ((double)used * K * N + (double)M * (K + N));
+    double best_t = 0;
+    int best = -1;
+    for (int i = 0; i < (int)(sizeof(kGmmCand) / sizeof(kGmmCand[0])); ++i) {
+        const GmmCand& c = kGmmCand[i];
+        const int64_t tiles = mt[c.bm == 32 ? 0 : c.bm == 64 ? 1 : c.bm == 128 ? 2 : 3] * ((N + c.bn - 1) / c.bn);
+        if (!grid_fits(tiles, c.threads)) continue;
+        const double run = tile_rounds_us(tiles, units, c.p, c.r, c.o);
+        const double mem = bytes / (c.bw * 1e6);
+        const double t = run * run * run * run + mem * mem * mem * mem;
+        if (best < 0 || t < best_t) {
+            best = i;
+            best_t = t;
+        }
+    }
+    return best;
 }
 
 }  // namespace cb

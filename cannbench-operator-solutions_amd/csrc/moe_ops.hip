@@ -4,7 +4,6 @@
 //   cb_quant_matmul                 (QuantMatmul)
 // plus the status strings.  Each entry point validates in the reference plugin's order, then
 // enqueues its kernels on the caller's stream without any allocation or host synchronisation.
-#include <cmath>
 #include <cstring>
 #include <cstdlib>
 #include <mutex>
@@ -100,7 +99,6 @@ void set_dynamic_lds_once(const void* kern, int bytes)
         (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
-static constexpr int kSkinnyMaxRows = 32;  // groups up to this many rows take the skinny core
 // The LDS core for prefill / dense groups: 256 x 256 tiles, 8 waves of 64 x 128, a 2-stage ring of
 // 128-deep stages.
 static constexpr int kLdsWM = 4, kLdsWN = 2, kLdsStages = 2, kLdsBK = 128;
@@ -115,68 +113,6 @@ static int xcd_split(int ntiles, int64_t E, int64_t tile_row_bytes)
     for (int P = 4; P >= 1; P >>= 1)
         if (ntiles % P == 0 && E % (8 / P) == 0 && (ntiles / P) * tile_row_bytes >= 1024) return P;
     return 0;
-}
-
-// ---- the dequant GEMM's choice of kernel -------------------------------------------------------
-// Estimated time in us of a BM x BN tile kernel over the call (tile_rounds_us: p us per 128 of K for a
-// tile alone on its CU, r in a full round of 256, o per tile); the bytes the call must move pass at
-// bw TB/s, partly hidden by the multiplications (the two times combine as the root of their
-// squares); f us per call.  The constants are fitted to
-// the measured times below; the 256 x 256 ring core and the skinny kernel (at most 32 rows per
-// group) are candidates like the others, so the rule compares like with like.
-//   us, by rows (dense 7168 x 4096)          us, by rows per expert (256 x 2048 x 7168)
-//                  24    300   1024  2048  4096       8     24    47    96    256
-//   32 x 64       18.3   38     87   165   321       836   912  1257  1971  4750
-//   64 x 128      23.2   24     44    84   161       705   782   829  1054  2019
-//   64 x 256      36     36     41    75   140       680   736   801   988  1764
-//   128 x 128     26     27     35    69   134       921   956  1003  1065  2068
-//   128 x 256     40     42     45    61   118       797   841   907   999  1716
-//   ring          (40)   69     78    98   101       840   800   830   930  1395
-//   skinny        55      -      -     -     -       624
-// With 2048 x 1024 weights 24 rows take 6.0 us (32 x 64) against 16.3 (skinny), 1024 rows 11.3
-// (64 x 128) against 28 (ring); 64 x 768 x 2048 with 96 / 200 rows per expert 34 / 44 (ring) against
-// 41 / 63 (64 x 256).
-struct DeqCand {
-    int bm, bn;
-    double p, r, o, bw, f;
-};
-enum { DEQ_RING = 5, DEQ_SKINNY = 6 };
-static constexpr DeqCand kDeqCand[] = {
-    {32, 64, 0.30, 0.152, 1.5, 5.2, 2.0},   {64, 128, 0.36, 0.31, 2.7, 6.8, 2.0},  {64, 256, 0.58, 0.54, 4.6, 6.55, 2.0},
-    {128, 128, 0.34, 0.486, 6.8, 6.5, 2.0}, {128, 256, 0.55, 0.87, 10.6, 6.5, 2.0}, {256, 256, 1.55, 1.55, 12.0, 12.0, 2.0},
-    {32, 256, 0.85, 0.30, 1.0, 6.3, 3.0},
-};
-
-static int pick_deq(const GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch, int max_rows, bool ring_ok)
-{
-    const double units = (double)((a.K + 127) / 128);
-    int64_t mt[4] = {0, 0, 0, 0}, used = 0, prev = 0;  // row tiles of 32, 64, 128 and 256 rows
-    for (int64_t g = 0; g < E; ++g) {
-        const int64_t rows = gl[g] - prev;
-        for (int j = 0; j < 4; ++j) mt[j] += (rows + (32 << j) - 1) >> (5 + j);
-        used += rows > 0;
-        prev = gl[g];
-    }
-    const double bytes = (double)batch * ((double)used * a.K * a.N + (double)a.M * (a.K + 2 * a.N));
-    double best_t = 0;
-    int best = -1;
-    for (int i = 0; i < (int)(sizeof(kDeqCand) / sizeof(kDeqCand[0])); ++i) {
-        const DeqCand& c = kDeqCand[i];
-        if (i == DEQ_SKINNY && max_rows > kSkinnyMaxRows) continue;
-        if (i == DEQ_RING && !ring_ok) continue;
-        const int64_t tiles = mt[c.bm == 32 ? 0 : c.bm == 64 ? 1 : c.bm == 128 ? 2 : 3] * ((a.N + c.bn - 1) / c.bn) * batch;
-        if (tiles > (1 << 24) && best >= 0) continue;
-        // the ring core's epilogue leaves out 32-row fragments without valid rows
-        const double o = i == DEQ_RING ? 2.0 + 10.0 * (double)mt[0] / (8.0 * (double)mt[3]) : c.o;
-        const double run = tile_rounds_us(tiles, units, c.p, c.r, o);
-        const double mem = bytes / (c.bw * 1e6);
-        const double t = c.f + std::sqrt(run * run + mem * mem);
-        if (best < 0 || t < best_t) {
-            best = i;
-            best_t = t;
-        }
-    }
-    return best;
 }
 
 template <int EPI>
@@ -198,13 +134,12 @@ static void launch_gemm(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch
         return;
     }
     if constexpr (EPI == EPI_DEQUANT) {
-        const int64_t rows = a.gt.max_rows;
         // 32-bit offsets within a tile's activation and output rows
         const bool tile_ok = 128 * a.K < 0x7fffffffLL && 256 * Ncols < 0x7fffffffLL && batch <= 65535;
         int pick = -1;
         if (tile_ok && g_overrides.gmm_tile > 0 && g_overrides.gmm_tile <= 5) pick = g_overrides.gmm_tile - 1;  // test hook
         else if (tile_ok && g_overrides.persistent_grid == 0)
-            pick = pick_deq(a, gl, E, batch, (int)rows, a.K >= 4 * PfCfg::BK || batch > 1);
+            pick = pick_deq(gl, E, a.M, a.K, a.N, batch, a.K >= 4 * PfCfg::BK || batch > 1);
         // otherwise the skinny kernel or the 256 x 256 cores below
         if (launch_deq_tile(pick, a, gl, E, batch, st)) return;
     }

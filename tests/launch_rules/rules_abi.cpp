@@ -4,4 +4,9 @@
 extern "C" {
 int rule_grid_fits(int64_t blocks, int64_t threads) { return cb::grid_fits(blocks, threads); }
 int64_t rule_dqsq_blocks(int64_t M, int64_t threads) { return cb::dqsq_blocks(M, threads); }
+int rule_pick_deq(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N, int64_t batch, int ring_ok)
+{
+    return cb::pick_deq(gl, E, M, K, N, batch, ring_ok);
+}
+int rule_pick_gmm(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N) { return cb::pick_gmm(gl, E, M, K, N); }
 }

@@ -22,6 +22,9 @@ def rules(tmp_path_factory):
     lib.rule_grid_fits.argtypes = [i64, i64]
     lib.rule_dqsq_blocks.argtypes = [i64, i64]
     lib.rule_dqsq_blocks.restype = i64
+    gl = ctypes.POINTER(i64)
+    lib.rule_pick_deq.argtypes = [gl, i64, i64, i64, i64, i64, ctypes.c_int]
+    lib.rule_pick_gmm.argtypes = [gl, i64, i64, i64, i64]
     return lib
 
 
@@ -35,3 +38,35 @@ def test_dqsq_grid(rules, threads):
         assert rules.rule_grid_fits(n, threads), (M, n)
     # below the limit: two rows each
     assert rules.rule_dqsq_blocks(131072, threads) == max(65536, 512 * (2048 // threads))
+
+
+# tile numbers of the rules: (rows, columns, threads)
+DEQ_TILES = [(32, 64, 256), (64, 128, 256), (64, 256, 256), (128, 128, 512), (128, 256, 512)]
+GMM_TILES = DEQ_TILES + [(256, 256, 512)]
+
+
+def _one_group(M):
+    return (ctypes.c_int64 * 1)(M)
+
+
+# outputs of at most 64 GB: rows up to the operators' limit with the narrowest vector columns, and wide ones
+BIG_SHAPES = [(M, n) for M in (1, 1 << 20, 1 << 27, (1 << 28) + 1, 1 << 29, 1 << 30, BIG)
+              for n in (8, 16, 48, 512, 8192) if M * n <= 1 << 35]
+
+
+@pytest.mark.parametrize("M,N", BIG_SHAPES)
+@pytest.mark.parametrize("K", [16, 64, 256])
+def test_tile_grids(rules, M, N, K):
+    """The tile that a rule picks fits a dispatch: 2^30 x 16 outputs are 2^24 tiles of 64 x 128 with 256
+    threads, one dispatch too many.  (A rule that finds no fitting tile names none, and the caller takes
+    the kernels that tile coarser or walk their tiles.)"""
+    tiles = lambda t: -(-M // t[0]) * -(-N // t[1])
+    if N % 16 == 0:
+        p = rules.rule_pick_deq(_one_group(M), 1, M, K, N, 1, K >= 256)
+        if 0 <= p < len(DEQ_TILES):
+            t = DEQ_TILES[p]
+            assert rules.rule_grid_fits(tiles(t), t[2]), (p, tiles(t))
+    p = rules.rule_pick_gmm(_one_group(M), 1, M, K, N)
+    if p >= 0:
+        t = GMM_TILES[p]
+        assert rules.rule_grid_fits(tiles(t), t[2]), (p, tiles(t))
