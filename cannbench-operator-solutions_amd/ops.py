@@ -61,8 +61,13 @@ def _dtype_code(dt):
     return _DTYPE_CODES.get(dt, -1)
 
 
+def _rereadable(group_list):
+    """group_list itself, or the list of its entries when it can be read only once (an iterator)."""
+    return group_list if hasattr(group_list, "__len__") else list(group_list)
+
+
 def _group_array(group_list, E, M, max_e):
-    """group_list as a host int64 array.array when it is a valid cumulative list (E entries, 1 to max_e
+    """group_list (rereadable) as a host int64 array.array when it is a valid cumulative list (E entries, 1 to max_e
     of them, non-decreasing from at least 0 up to M), else None: the caller's element-by-element checks
     then name the fault (or convert entries that only int() takes).  256 experts take 4.6 us here, 32 in
     the Python loops."""
@@ -164,6 +169,7 @@ def grouped_matmul_swiglu_quant_meta(x, weight, weight_scale, x_scale, group_lis
 
 
 def _validate_group_list(prefix, group_list, E, M, max_e):
+    group_list = _rereadable(group_list)
     gl = _group_array(group_list, E, M, max_e)
     if gl is not None:
         return gl
@@ -413,6 +419,7 @@ def grouped_matmul_quant(x, weight, weight_scale, x_scale, group_list):
     _check(x_scale.numel() == M, f"{name}: x_scale must have M elements")
     _check(weight_scale.dim() == 2 and weight_scale.size(0) == E and weight_scale.size(1) == N,
            f"{name}: weight_scale must be [E, N]")
+    group_list = _rereadable(group_list)
     gl = _group_array(group_list, E, M, L.CB_MAX_EXPERTS)
     if gl is None:
         gl = [int(v) for v in group_list]

@@ -166,3 +166,31 @@ def test_grouped_matmul_checks_and_outputs(cb):
     assert len(outs) == 1 and outs[0].shape == (0, 3)
     views = cb.ops.grouped_matmul_meta(x, torch.zeros(2, 3, 8, dtype=f), [2, 5], transpose_weight=True)
     assert [v.shape for v in views] == [(2, 3), (3, 3)]
+
+
+class _IntOnly:
+    """A value that int() takes and operator.index() does not."""
+
+    def __init__(self, v):
+        self.v = v
+
+    def __int__(self):
+        return self.v
+
+
+@pytest.mark.parametrize("entries", [iter, lambda v: (x for x in v), lambda v: map(float, v), lambda v: map(_IntOnly, v),
+                                     tuple, lambda v: torch.tensor(v, dtype=torch.float64)],
+                         ids=["iterator", "generator", "floats", "int_only", "tuple", "float_tensor"])
+def test_group_list_forms(cb, entries):
+    """A group list is any iterable of values int() takes, one that can be read only once included: a valid
+    one passes every check (and stops at the missing device), an invalid one is named for what it is."""
+    gmsq = lambda gl: cb.grouped_matmul_swiglu_quant(i8(4, 8), i8(2, 8, 16), f32(2, 16), f32(4), gl)
+    down = lambda gl: cb.grouped_matmul_quant(i8(4, 8), i8(2, 8, 16), f32(2, 16), f32(4), gl)
+    raw = lambda gl: cb.grouped_matmul_int32(i8(4, 8), i8(2, 8, 16), gl)
+    for fn in (gmsq, down, raw):
+        with pytest.raises(RuntimeError, match="ROCm device"):
+            fn(entries([2, 4]))
+        with pytest.raises(RuntimeError, match="must equal M"):
+            fn(entries([1, 3]))
+        with pytest.raises(RuntimeError, match="cumsum"):
+            fn(entries([3, 2]))
