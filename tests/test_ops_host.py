@@ -194,3 +194,34 @@ def test_group_list_forms(cb, entries):
             fn(entries([1, 3]))
         with pytest.raises(RuntimeError, match="cumsum"):
             fn(entries([3, 2]))
+
+
+class _Marked(torch.Tensor):
+    """A tensor subclass as a caller may use one."""
+
+
+def _marked(t):
+    return t.as_subclass(_Marked)
+
+
+def test_outputs_of_subclass_inputs_are_plain_tensors(cb):
+    """The operators allocate plain tensors, whatever class the inputs have (empty inputs and the shape
+    functions return without a device); only xOut, created like x1, follows its class."""
+    bf, m8 = torch.zeros(4, 8, dtype=torch.bfloat16), torch.zeros(4, 8, dtype=torch.int8)
+    ops = cb.ops
+    outs = [
+        *cb.grouped_matmul_swiglu_quant(_marked(i8(0, 8)), i8(2, 8, 16), f32(2, 16), f32(0), [0, 0]),
+        *ops.grouped_matmul_swiglu_quant_meta(_marked(m8), i8(2, 8, 16), f32(2, 16), f32(4), [2, 4]),
+        cb.grouped_matmul_quant(_marked(i8(0, 8)), i8(2, 8, 16), f32(2, 16), f32(0), [0, 0]),
+        cb.grouped_matmul_int32(_marked(i8(0, 8)), i8(2, 8, 16), [0, 0]),
+        ops.quant_matmul_meta(_marked(m8), i8(8, 16), f32(16)),
+        *cb.grouped_matmul(_marked(bf[:0]), torch.zeros(1, 8, 16, dtype=torch.bfloat16), [0], split_item=2),
+        *ops.grouped_matmul_meta(_marked(bf), torch.zeros(1, 8, 16, dtype=torch.bfloat16), [4], split_item=2),
+        *ops.dynamic_quant_meta(_marked(bf)),
+        *ops.add_rms_norm_dynamic_quant_meta(_marked(bf), bf, bf[0].clone(), 1e-6)[::2],
+        *ops.moe_re_routing_meta(_marked(bf), _marked(torch.ones(2, 2, dtype=torch.int32))),
+        ops.moe_finalize_routing_meta(_marked(bf), torch.zeros(4, dtype=torch.int32)),
+        *ops.dequant_swiglu_quant_meta(_marked(bf)),
+        *ops.moe_gating_top_k_softmax_meta(_marked(bf.float()), k=2),
+    ]
+    assert [type(o) for o in outs] == [torch.Tensor] * len(outs)
