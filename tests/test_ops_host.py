@@ -225,3 +225,21 @@ def test_outputs_of_subclass_inputs_are_plain_tensors(cb):
         *ops.moe_gating_top_k_softmax_meta(_marked(bf.float()), k=2),
     ]
     assert [type(o) for o in outs] == [torch.Tensor] * len(outs)
+
+
+def test_stream_handle_without_the_raw_getters(cb, monkeypatch):
+    """Where torch lacks the two internal functions that read the stream handle, the public current_stream()
+    gives it."""
+    import types
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=4711))
+    assert cb.ops._stream_reader(types.SimpleNamespace())() == 4711
+    raw = types.SimpleNamespace(_cuda_getDevice=lambda: 3, _cuda_getCurrentRawStream=lambda d: 100 + d)
+    assert cb.ops._stream_reader(raw)() == 103
+
+
+@pytest.mark.gpu
+def test_stream_handle_is_the_current_stream(cb):
+    side = torch.cuda.Stream()
+    assert cb.ops._stream() == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert cb.ops._stream() == side.cuda_stream
