@@ -812,14 +812,16 @@ __device__ __forceinline__ void pf_epilogue(const GemmArgs& a, uint8_t* smem, v1
 // published.  No workgroup waits for its row tile's other column tiles, so a late one (a slow
 // weight line, an HBM-bound tile of a small expert) costs nothing until it is a whole tile late.
 //
-// Fragment rows fm >= nv hold no valid rows (uniform, as in the K loop): publish leaves their old
-// activations in place, unread, and the requant stops before them.  A tile of 47 rows otherwise
-// spends three quarters of both on rows that are never stored: 256 experts of 7168 x 4096 with 47
-// rows each 1380 -> 1323 us, 64 experts of 2048 x 1536 with 47 rows 78.8 -> 66.9.
+// SKIP (an instance of its own, gmsq_skips_empty of launch_rules.hpp chooses): fragment rows fm >= nv
+// hold no valid rows (uniform, as in the K loop); publish leaves their old activations in place, unread,
+// and the requant stops before them.  A tile of 47 rows otherwise spends three quarters of both on rows
+// that are never stored.  The branches and the second set of activations they need cost a full tile
+// 1 to 2%, and copies of both steps for full tiles inside one kernel cost more than that.
 //
 // publish (after the K loop): SwiGLU from the accumulators into act, row maxima of |act| across
 // the lanes (DPP) and the two waves sharing the rows (LDS), one agent-scope atomicMax per (row,
 // tile), then one arrival on the row tile's counter once every maximum has completed.
+template <bool SKIP>
 __device__ __forceinline__ void pf_publish(const GemmArgs& a, uint8_t* smem, v16i (&acc)[4][4], const PfTile& t,
                                            const int par, const int nv, float (&act)[4][2][16])
 {
@@ -841,10 +843,11 @@ __device__ __forceinline__ void pf_publish(const GemmArgs& a, uint8_t* smem, v16
     // VGPRs they occupy during the next K loop are then not needed on top of this step's own), and
     // moved to VGPRs at the end.
     float tmp[4][2][16];
+    float(&v)[4][2][16] = SKIP ? tmp : act;
     // lane (h, c) of fragment (fm, fn) holds rows (2 fm + wm) * 32 + 8 (r / 4) + 4 h + r % 4, column c
 #pragma unroll
     for (int fm = 0; fm < 4; ++fm) {
-        if (fm && fm >= nv) continue;
+        if (SKIP && fm && fm >= nv) continue;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int row = (2 * fm + wm) * 32 + 8 * q + 4 * h;
@@ -853,7 +856,7 @@ __device__ __forceinline__ void pf_publish(const GemmArgs& a, uint8_t* smem, v16
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
-                    tmp[fm][j][4 * q + i] = to_agpr(swiglu((float)acc_read(acc[fm][j][4 * q + i]),
+                    v[fm][j][4 * q + i] = to_agpr(swiglu((float)acc_read(acc[fm][j][4 * q + i]),
                                                            (float)acc_read(acc[fm][j + 2][4 * q + i]), xs4[i], wsg[j], wsu[j]));
         }
     }
@@ -863,12 +866,12 @@ __device__ __forceinline__ void pf_publish(const GemmArgs& a, uint8_t* smem, v16
     // row_bcast:15 into rows 1 and 3: lanes 16..31 and 48..63 end with their half-wave's maximum.
 #pragma unroll
     for (int fm = 0; fm < 4; ++fm) {
-        if (fm && fm >= nv) continue;
+        if (SKIP && fm && fm >= nv) continue;
         u32 m[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const u32 u0 = __float_as_uint(from_agpr(tmp[fm][0][r])) & 0x7fffffffu;
-            const u32 u1 = __float_as_uint(from_agpr(tmp[fm][1][r])) & 0x7fffffffu;
+            const u32 u0 = __float_as_uint(from_agpr(v[fm][0][r])) & 0x7fffffffu;
+            const u32 u1 = __float_as_uint(from_agpr(v[fm][1][r])) & 0x7fffffffu;
             const u32 v0 = u0 > 0x7f800000u ? 0u : u0, v1 = u1 > 0x7f800000u ? 0u : u1;
             m[r] = v0 > v1 ? v0 : v1;
         }
@@ -901,22 +904,23 @@ __device__ __forceinline__ void pf_publish(const GemmArgs& a, uint8_t* smem, v16
     if (tid == 0) pf_arrive(e.arrive + t.mt);
 #pragma unroll
     for (int fm = 0; fm < 4; ++fm) {
-        if (fm && fm >= nv) continue;
+        if (SKIP && fm && fm >= nv) continue;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) act[fm][j][r] = from_agpr(tmp[fm][j][r]);
+            for (int r = 0; r < 16; ++r) act[fm][j][r] = from_agpr(v[fm][j][r]);
     }
 }
 
 // The pending requant of a workgroup's previous tile (has: one is pending).
+template <bool SKIP>
 struct PfDefer {
     float (&act)[4][2][16];  // its activations
     const GemmArgs& a;
     uint8_t* smem;
     int nt;       // its column tile
     u32 target;   // arrivals that complete a row tile's maxima
-    int nv;       // its fragment rows with valid rows
+    int nv;       // its fragment rows with valid rows (SKIP)
     bool has;
     PfTile t;     // its row tile
 
@@ -988,7 +992,7 @@ struct PfDefer {
             }
 #pragma unroll
             for (int fm = 0; fm < 4; ++fm) {
-                if (fm && fm >= nv) break;
+                if (SKIP && fm && fm >= nv) break;
 #pragma unroll
                 for (int qp = 0; qp < 2; ++qp) {
                     const v4f ia = *(const CB_LDS v4f*)(inv_l + (2 * fm + wm) * 32 + 16 * qp + 4 * h);
@@ -1008,7 +1012,7 @@ struct PfDefer {
         }
 #pragma unroll
         for (int fm = 0; fm < 4; ++fm) {
-            if (fm && fm >= nv) break;
+            if (SKIP && fm && fm >= nv) break;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const v4f inv4 = *(const CB_LDS v4f*)(inv_l + (2 * fm + wm) * 32 + 8 * q + 4 * h);
@@ -1027,10 +1031,11 @@ struct PfDefer {
 // row tile mt are final once its ntl column tiles have counted at arrive[mt].  GATHER: activation rows
 // through the row index.
 // DEFER: each tile's requant waits until the workgroup's next K loop is done (PfDefer); needs the
-// K loop that carries the next tile's prologue (K of at least kPfDeferMinStages stages).
+// K loop that carries the next tile's prologue (K of at least kPfDeferMinStages stages).  SKIP (with
+// DEFER): see pf_publish.
 constexpr int kPfDeferMinStages = 4;
 
-template <bool GATHER, bool DEFER>
+template <bool GATHER, bool DEFER, bool SKIP>
 __global__ __launch_bounds__(256, 1) void gmsq_prefill_kernel(const GemmArgs a)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -1076,7 +1081,7 @@ __global__ __launch_bounds__(256, 1) void gmsq_prefill_kernel(const GemmArgs a)
     }
     bool first = true;
     float act[4][2][16];  // DEFER: the pending tile's activations
-    PfDefer def{act, a, smem, 0, target, 0, false, cur_t};
+    PfDefer<SKIP> def{act, a, smem, 0, target, 0, false, cur_t};
     for (; q < rounds; q += pl.slots) {
         // opaque: the DMA offsets derived from these (every stage of every loop variant) are
         // computed per tile, not hoisted out of the tile loop and spilled
@@ -1126,7 +1131,7 @@ __global__ __launch_bounds__(256, 1) void gmsq_prefill_kernel(const GemmArgs a)
             else if (nv == 1) pf_kloop<1, true, GATHER>(cur, nxt, offs, nk, rb, smem, a_rd, b_rd, acc, wave, first);
             else pf_kloop<0, true, GATHER>(cur, nxt, offs, nk, rb, smem, a_rd, b_rd, acc, wave, first);
             def.run();
-            pf_publish(a, smem, acc, cur_t, par, nv, act);
+            pf_publish<SKIP>(a, smem, acc, cur_t, par, nv, act);
             def.nv = nv;
             def.has = true;
             def.t = cur_t;

@@ -26,6 +26,30 @@ inline int64_t dqsq_blocks(int64_t M, int64_t threads)
     return want < most ? want : most;
 }
 
+// Whether the GroupedMatmulSwigluQuant prefill kernel leaves out the publish and requant of 32-row
+// fragments without valid rows (its SKIP instance): yes when no 256-row tile is full enough to lose by it,
+// or when the empty fragments outweigh what full tiles lose and the tiles fill at least two rounds of
+// the grid (below that the call takes as long as its full tiles).  Measured gain of SKIP, by valid
+// share of the fragments:
+//   256 x 7168 x 4096:  47 rows per expert (0.25) 1.035, 128 rows (0.5) 1.037, 192 (0.75) 1.016,
+//                       256 (1.0) 0.99, Zipf 128 on average (0.43) 1.025, Zipf 512 (0.81) level
+//   128 x 2048 x 2048:  47 rows 1.18, 128 rows 1.08, 300 rows (0.62) 0.93, 288 rows (0.56) 0.93
+//   64 x 2048 x 1536:   47 rows 1.22, 300 rows 0.95; 16 x 4096 x 2048, Zipf 64 (under two rounds) 0.97
+// Experts of just over 256 rows (a full tile and a nearly empty one, valid share 9/16 at least) lose
+// most: a workgroup meets the same kind of tile in every round, and the early ones run out of step.
+inline bool gmsq_skips_empty(const int64_t* gl, int64_t E, int64_t ntl, int64_t grid)
+{
+    int64_t frags = 0, tiles = 0, max_rows = 0, prev = 0;
+    for (int64_t g = 0; g < E; ++g) {
+        const int64_t rows = gl[g] - prev;
+        frags += (rows + 31) / 32;
+        tiles += (rows + 255) / 256;
+        max_rows = rows > max_rows ? rows : max_rows;
+        prev = gl[g];
+    }
+    return max_rows <= 192 || (2 * frags < 9 * tiles && tiles * ntl >= 2 * grid);
+}
+
 // Time model of a tiled GEMM for the rules that choose a tile: a tile alone on its CU takes p us per
 // K unit and o us for its prologue and epilogue; with a tile on each of the 256 CUs a round takes r us
 // per K unit and o us (r above p: the CUs share L2 and fabric bandwidth; below: several workgroups

@@ -328,10 +328,13 @@ static int gmsq_impl(const int8_t* x, int64_t x_rows, const int32_t* row_index, 
         const int grid = (ntl == 16 && cus >= 256) ? 256 : (cus / ntl) * ntl;
         const bool gather = row_index != nullptr;
         const bool defer = (K + PfCfg::BK - 1) / PfCfg::BK >= kPfDeferMinStages;
-        const void* main_k = gather ? (defer ? (const void*)gmsq_prefill_kernel<true, true>
-                                             : (const void*)gmsq_prefill_kernel<true, false>)
-                                    : (defer ? (const void*)gmsq_prefill_kernel<false, true>
-                                             : (const void*)gmsq_prefill_kernel<false, false>);
+        const bool skip = gmsq_skips_empty(group_list, E, ntl, grid);
+        const void* main_k = !defer   ? (gather ? (const void*)gmsq_prefill_kernel<true, false, false>
+                                                : (const void*)gmsq_prefill_kernel<false, false, false>)
+                             : gather ? (skip ? (const void*)gmsq_prefill_kernel<true, true, true>
+                                              : (const void*)gmsq_prefill_kernel<true, true, false>)
+                                      : (skip ? (const void*)gmsq_prefill_kernel<false, true, true>
+                                              : (const void*)gmsq_prefill_kernel<false, true, false>);
         const void* fix_k =
             gather ? (const void*)gmsq_prefill_fixup_kernel<true> : (const void*)gmsq_prefill_fixup_kernel<false>;
         int resident = 0;

@@ -9,4 +9,8 @@ int rule_pick_deq(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N,
     return cb::pick_deq(gl, E, M, K, N, batch, ring_ok);
 }
 int rule_pick_gmm(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N) { return cb::pick_gmm(gl, E, M, K, N); }
+int rule_gmsq_skips_empty(const int64_t* gl, int64_t E, int64_t ntl, int64_t grid)
+{
+    return cb::gmsq_skips_empty(gl, E, ntl, grid);
+}
 }

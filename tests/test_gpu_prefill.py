@@ -214,3 +214,28 @@ def test_int32_core_tile_bytes_past_4gib(cb):
         np.testing.assert_array_equal(c[r0:r0 + 256].cpu().numpy(), ref, err_msg=f"rows {r0}:{r0 + 256}")
     del c
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("y_offset", [0, 4, 1])  # 8-byte, dword and byte stores
+@pytest.mark.parametrize("counts,K,N", [
+    ([40, 7, 190, 33], 320, 288),               # no tile is nearly full: the instance without the empty fragments
+    ([300] + [40] * 33 + [1, 0, 64], 256, 4096),  # the same beside a full tile and two nearly empty ones
+])
+def test_prefill_instances_agree(cb, orc, counts, K, N, y_offset):
+    """The prefill kernel has an instance that leaves out empty 32-row fragments and one that does not; the
+    call's groups choose.  A row's result depends on its own group alone: every group computed beside a group
+    of 256 full rows that makes the call take the other instance gives the same bits, and the call meets the
+    oracle."""
+    x, w, ws, xs, gl = _inputs(counts, K, N, sum(counts))
+    y, ys, _ = _run_raw(cb, x, w, ws, xs, gl, y_offset)
+    yr, ysr = orc.gmsq(x.cpu().numpy(), w.cpu().numpy(), ws.cpu().numpy(), xs.cpu().numpy(), np.array(gl))
+    assert np.abs(y.cpu().numpy().astype(int) - yr).max() <= 1
+    np.testing.assert_allclose(ys.cpu().numpy(), ysr, rtol=1e-5)
+    full = rand_i8((256, K), cpu_gen(1))
+    for g in {0, 1, len(counts) - 1}:
+        a, b = (gl[g - 1] if g else 0), gl[g]
+        if b - a == 0:
+            continue
+        yo, yso, _ = _run_raw(cb, torch.cat([x[a:b], full]), torch.stack([w[g], w[g]]), torch.stack([ws[g], ws[g]]),
+                              torch.cat([xs[a:b], xs.new_full((256,), 0.01)]), [b - a, b - a + 256], y_offset)
+        assert torch.equal(yo[:b - a], y[a:b]) and torch.equal(yso[:b - a], ys[a:b])

@@ -25,6 +25,7 @@ def rules(tmp_path_factory):
     gl = ctypes.POINTER(i64)
     lib.rule_pick_deq.argtypes = [gl, i64, i64, i64, i64, i64, ctypes.c_int]
     lib.rule_pick_gmm.argtypes = [gl, i64, i64, i64, i64]
+    lib.rule_gmsq_skips_empty.argtypes = [gl, i64, i64, i64]
     return lib
 
 
@@ -70,3 +71,25 @@ def test_tile_grids(rules, M, N, K):
     if p >= 0:
         t = GMM_TILES[p]
         assert rules.rule_grid_fits(tiles(t), t[2]), (p, tiles(t))
+
+
+def _gl(counts):
+    ends, s = [], 0
+    for c in counts:
+        s += c
+        ends.append(s)
+    return (ctypes.c_int64 * len(ends))(*ends)
+
+
+@pytest.mark.parametrize("counts,skips", [
+    ([33] * 64, True), ([47] * 256, True), ([192] * 8, True),          # no tile full enough to lose
+    ([256] * 256, False), ([224] * 64, False), ([512] * 64, False),    # full tiles
+    ([257] * 128, False), ([288] * 128, False), ([300] * 256, False),  # a full and a nearly empty tile each
+    ([300] + [40] * 255, True),                                        # many small groups beside a full tile
+    ([300] + [40] * 15, False),                                        # the same, under two rounds of the grid
+    ([0] * 200 + [0, 40, 0], True),
+])
+def test_gmsq_skip_rule(rules, counts, skips):
+    """Leaving out the empty fragments is taken where it gains (groups far below a tile) and not where it loses
+    (full tiles; groups of just over a tile)."""
+    assert bool(rules.rule_gmsq_skips_empty(_gl(counts), len(counts), 16, 256)) is skips
