@@ -151,10 +151,10 @@ __device__ __forceinline__ PfScales gpf_scales(const GemmArgs& a, const GpfTile&
 
 // The dequant epilogue of one tile from the accumulators.  Lane (h = lane / 32, c = lane % 32) of
 // fragment (fm, fn) holds rows (2 fm + wm) * 32 + 8 (r / 4) + 4 h + r % 4, column
-// tcol(fn) + c with tcol(fn) = 128 (fn / 2) + 64 wn + 32 (fn % 2).  FULL: every fragment row has valid
-// rows; otherwise the rows fm >= nv have none and are left out (a copy of its own, as the branches
-// cost full tiles 1 to 2%): 64 experts of 768 x 2048 with 96 rows each 38.5 -> 34.0 us, 256 experts
-// of 2048 x 7168 with 47 rows 840 -> 780.
+// tcol(fn) + c with tcol(fn) = 128 (fn / 2) + 64 wn + 32 (fn % 2).  FULL: all fragment rows, with or
+// without valid rows (the resource drops the stores of the others); otherwise the rows fm >= nv have
+// none and are left out (a copy of its own, as the branches cost full tiles 1 to 2%): 64 experts of
+// 768 x 2048 with 96 rows each 38.5 -> 34.0 us, 256 experts of 2048 x 7168 with 47 rows 840 -> 780.
 template <bool SIMPLE, bool FULL>
 __device__ __forceinline__ void gpf_epilogue(const GemmArgs& a, uint8_t* smem, v16i (&acc)[4][4], const GpfTile& t,
                                              const int par, const int nv)
@@ -239,8 +239,9 @@ __device__ __forceinline__ void gpf_epilogue(const GemmArgs& a, uint8_t* smem, v
 
 // Persistent launch: gridDim.x workgroups (at most one per CU) walk the launch order's slots.
 // Batch 1, K of at least 4 stages, N a multiple of 8 and the output 16-byte aligned (16-byte
-// stores), bf16 / fp16 out.
-template <bool SIMPLE>
+// stores), bf16 / fp16 out.  SKIP: tiles with empty fragment rows leave them out of the epilogue
+// (ring_skips_empty of launch_rules.hpp chooses).
+template <bool SIMPLE, bool SKIP>
 __global__ __launch_bounds__(256, 1) void gpf_dequant_kernel(const GemmArgs a)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -289,7 +290,7 @@ __global__ __launch_bounds__(256, 1) void gpf_dequant_kernel(const GemmArgs a)
         else if (nv == 2) pf_kloop<2, true, false>(cur, nxt, offs, nk, rb, smem, a_rd, b_rd, acc, wave, first);
         else if (nv == 1) pf_kloop<1, true, false>(cur, nxt, offs, nk, rb, smem, a_rd, b_rd, acc, wave, first);
         else pf_kloop<0, true, false>(cur, nxt, offs, nk, rb, smem, a_rd, b_rd, acc, wave, first);
-        if (nv >= 4) gpf_epilogue<SIMPLE, true>(a, smem, acc, cur_t, par, nv);
+        if (!SKIP || nv >= 4) gpf_epilogue<SIMPLE, true>(a, smem, acc, cur_t, par, nv);
         else gpf_epilogue<SIMPLE, false>(a, smem, acc, cur_t, par, nv);
         if (has_nxt) put_scales(nsc, par ^ 1);
         // every wave is past this epilogue's scale reads (and the next scales are written) before

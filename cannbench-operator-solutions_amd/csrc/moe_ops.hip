@@ -168,13 +168,16 @@ static void launch_gemm(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch
             256 * Ncols * 2 < 0x7fffffffLL) {
             const EpiArgs& e = a.epi;
             const bool simple = !e.has_offset && e.bias_kind == BIAS_NONE && e.out_bf16;
-            const void* kern = simple ? (const void*)gpf_dequant_kernel<true> : (const void*)gpf_dequant_kernel<false>;
+            const bool skip = ring_skips_empty(gl, E);
+            const void* kern = simple ? (skip ? (const void*)gpf_dequant_kernel<true, true>
+                                              : (const void*)gpf_dequant_kernel<true, false>)
+                                      : (skip ? (const void*)gpf_dequant_kernel<false, true>
+                                              : (const void*)gpf_dequant_kernel<false, false>);
             set_dynamic_lds_once(kern, kGpfLds);
             // both launch orders spread the valid slots over up to a round of 256: launch the whole
             // grid (a grid of `blocks` workgroups walked several tiles each while others had none)
-            const dim3 grid((unsigned)pg);
-            if (simple) hipLaunchKernelGGL(gpf_dequant_kernel<true>, grid, dim3(256), kGpfLds, st, a);
-            else hipLaunchKernelGGL(gpf_dequant_kernel<false>, grid, dim3(256), kGpfLds, st, a);
+            void* args[] = {(void*)&a};
+            (void)hipLaunchKernel(kern, dim3((unsigned)pg), dim3(256), args, kGpfLds, st);  // checked by the caller
             return;
         }
     }

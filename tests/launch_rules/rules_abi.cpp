@@ -13,4 +13,5 @@ int rule_gmsq_skips_empty(const int64_t* gl, int64_t E, int64_t ntl, int64_t gri
 {
     return cb::gmsq_skips_empty(gl, E, ntl, grid);
 }
+int rule_ring_skips_empty(const int64_t* gl, int64_t E) { return cb::ring_skips_empty(gl, E); }
 }

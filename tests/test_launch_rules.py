@@ -26,6 +26,7 @@ def rules(tmp_path_factory):
     lib.rule_pick_deq.argtypes = [gl, i64, i64, i64, i64, i64, ctypes.c_int]
     lib.rule_pick_gmm.argtypes = [gl, i64, i64, i64, i64]
     lib.rule_gmsq_skips_empty.argtypes = [gl, i64, i64, i64]
+    lib.rule_ring_skips_empty.argtypes = [gl, i64]
     return lib
 
 
@@ -93,3 +94,12 @@ def test_gmsq_skip_rule(rules, counts, skips):
     """Leaving out the empty fragments is taken where it gains (groups far below a tile) and not where it loses
     (full tiles; groups of just over a tile)."""
     assert bool(rules.rule_gmsq_skips_empty(_gl(counts), len(counts), 16, 256)) is skips
+
+
+@pytest.mark.parametrize("counts,skips", [
+    ([33] * 64, True), ([129] * 16, True), ([256] * 8, True), ([224, 7, 0, 256], True),  # one tile per group
+    ([274] * 256, False), ([336] * 64, False), ([571] * 64, False),  # a full and a lighter tile in each group
+    ([600] + [40] * 31, True),                                       # mostly empty fragments
+])
+def test_ring_skip_rule(rules, counts, skips):
+    assert bool(rules.rule_ring_skips_empty(_gl(counts), len(counts))) is skips
