@@ -352,7 +352,7 @@ extern "C" int cb_grouped_matmul(const void* x, const void* weight, const void* 
         const int tile = g_overrides.gmm_tile;
         int pick = -1;
         if (tile != 128 && 256 * K * 2 < (1LL << 31) && 256 * N * 2 < (1LL << 31) && aligned(y, 16))  // 16-byte stores
-            pick = tile >= 1 && tile <= 6 ? tile - 1 : pick_gmm(group_list, E, M, K, N);
+            pick = tile >= 1 && tile <= 6 ? tile - 1 : pick_gmm(group_list, E, M, K, N, rule_cus());
         switch (pick) {
             case 0: launch_gmm_tile<GmmT0>(a, group_list, E, st); return check_launch();
             case 1: launch_gmm_tile<GmmT1>(a, group_list, E, st); return check_launch();

@@ -83,6 +83,16 @@ struct TestOverrides {
 };
 extern thread_local TestOverrides g_overrides;
 
+// Compute units of the current device (cached per device), 0 or less where they cannot be read.
+int device_cus();
+
+// The CU count for the rules that choose a tile.
+inline int rule_cus()
+{
+    const int cus = device_cus();
+    return cus > 0 ? cus : 256;
+}
+
 // Raise a kernel's dynamic LDS limit once per (kernel, device): the attribute belongs to the kernel as
 // loaded on the current device, so a process driving several GPUs sets it on each.
 void set_dynamic_lds_once(const void* kern, int bytes);

@@ -79,14 +79,14 @@ inline bool ring_skips_empty(const int64_t* gl, int64_t E)
 }
 
 // Time model of a tiled GEMM for the rules that choose a tile: a tile alone on its CU takes p us per
-// K unit and o us for its prologue and epilogue; with a tile on each of the 256 CUs a round takes r us
+// K unit and o us for its prologue and epilogue; with a tile on each of the cus CUs a round takes r us
 // per K unit and o us (r above p: the CUs share L2 and fabric bandwidth; below: several workgroups
 // per CU hide each other's latency).
-inline double tile_rounds_us(int64_t tiles, double units, double p, double r, double o)
+inline double tile_rounds_us(int64_t tiles, double units, double p, double r, double o, int64_t cus)
 {
     const double alone = units * p + o, full = units * r + o;
-    if (tiles < 256 && full > alone) return alone + (full - alone) * (double)tiles / 256;
-    const double t = (double)((tiles + 255) / 256) * full;
+    if (tiles < cus && full > alone) return alone + (full - alone) * (double)tiles / (double)cus;
+    const double t = (double)((tiles + cus - 1) / cus) * full;
     return t > alone ? t : alone;
 }
 
@@ -94,37 +94,46 @@ inline double tile_rounds_us(int64_t tiles, double units, double p, double r, do
 // Estimated time in us of a BM x BN tile kernel over the call (tile_rounds_us: p us per 128 of K for a
 // tile alone on its CU, r in a full round of 256, o per tile); the bytes the call must move pass at
 // bw TB/s, partly hidden by the multiplications (the two times combine as the root of their
-// squares); f us per call.  The constants are fitted to
-// the measured times below; the 256 x 256 ring core and the skinny kernel (at most 32 rows per
-// group) are candidates like the others, so the rule compares like with like.
-//   us, by rows (dense 7168 x 4096)          us, by rows per expert (256 x 2048 x 7168)
+// squares: powers of 3 and 4 fit worse); f us per call.  The
+// skinny kernel (at most 32 rows per group, in one or two blocks of 16), the 256 x 256 ring core (more
+// than 32 rows, batch 1, K of at least 256) and the 8-wave 256 x 256 kernel (more than 32 rows, other
+// batches and K) are candidates like the others.  Their constants are fits (bw and f need not be physical)
+// to 1700 shapes, 1 to 65536 rows, K 64 to 10240, N 64 to 16384, 1 to 256 groups, 1 to 32 batches, on
+// which every candidate was timed: the choice is 1.4% off the fastest on average.  Against taking no
+// tile at all one shape in a hundred loses more than 2% (1149 x 4672 x 14400, 129 against 117 us); with
+// the ring at 1.55 us per 128 of K and its constants for the 8-wave kernel too it was one in twenty,
+// up to 40% (1614 x 3648 x 12288, 111 against 95; 11288 x 208 x 1088, 19 against 14).  Measured:
+//   us, by rows (dense 7168 x 4096)          us, by rows per expert (256 x 2048 x 7168, drawn unevenly)
 //                  24    300   1024  2048  4096       8     24    47    96    256
-//   32 x 64       18.3   38     87   165   321       836   912  1257  1971  4750
-//   64 x 128      23.2   24     44    84   161       705   782   829  1054  2019
-//   64 x 256      36     36     41    75   140       680   736   801   988  1764
-//   128 x 128     26     27     35    69   134       921   956  1003  1065  2068
-//   128 x 256     40     42     45    61   118       797   841   907   999  1716
-//   ring          (40)   69     78    98   101       840   800   830   930  1395
-//   skinny        55      -      -     -     -       624
+//   32 x 64       19.2   39     96   189   379       803    -     -     -      -
+//   64 x 128      23.5   25     47    90   182       677   777   822  1054  2076
+//   64 x 256      36     36     47    82   164       656   723   794   984  1766
+//   128 x 128     26     28     37    74   152       910   954   993  1080  2120
+//   128 x 256     42     43     49    65   131       787   830   894   988  1749
+//   ring           -     67    101   104   105        -    752   817   917  1403
+//   skinny        52      -      -     -     -       615
 // With 2048 x 1024 weights 24 rows take 6.0 us (32 x 64) against 16.3 (skinny), 1024 rows 11.3
 // (64 x 128) against 28 (ring); 64 x 768 x 2048 with 96 / 200 rows per expert 34 / 44 (ring) against
-// 41 / 63 (64 x 256).
+// 41 / 63 (64 x 256).  8-wave kernel: 11288 x 208 x 1088 13.7 against 19.2 (64 x 256), 32 x (94 x 832 x
+// 1280) 14.3 against 18.9 (64 x 128).
 inline constexpr int kSkinnyMaxRows = 32;  // groups up to this many rows can take the skinny core
 
 struct DeqCand {
     int bm, bn, threads;  // threads 0: the launch does not grow with the number of tiles
     double p, r, o, bw, f;
+    double e;  // share of p and r that a tile takes whatever its valid rows; the rest goes with its valid 32-row fragments
 };
-enum { DEQ_RING = 5, DEQ_SKINNY = 6 };
+enum { DEQ_RING = 5, DEQ_SKINNY = 6, DEQ_LDS = 7, DEQ_SKINNY2 = 8 };  // 6, 8: one and two blocks of 16 rows
 inline constexpr DeqCand kDeqCand[] = {
-    {32, 64, 256, 0.30, 0.152, 1.5, 5.2, 2.0},   {64, 128, 256, 0.36, 0.31, 2.7, 6.8, 2.0},
-    {64, 256, 256, 0.58, 0.54, 4.6, 6.55, 2.0},  {128, 128, 512, 0.34, 0.486, 6.8, 6.5, 2.0},
-    {128, 256, 512, 0.55, 0.87, 10.6, 6.5, 2.0}, {256, 256, 0, 1.55, 1.55, 12.0, 12.0, 2.0},
-    {32, 256, 0, 0.85, 0.30, 1.0, 6.3, 3.0},
+    {32, 64, 256, 0.30, 0.152, 1.5, 5.2, 2.0, 1.0},   {64, 128, 256, 0.36, 0.31, 2.7, 6.8, 2.0, 1.0},
+    {64, 256, 256, 0.63, 0.58, 4.9, 6.9, 1.85, 1.0},  {128, 128, 512, 0.34, 0.486, 6.8, 6.5, 2.0, 1.0},
+    {128, 256, 512, 0.55, 0.87, 10.6, 6.5, 2.0, 1.0}, {256, 256, 0, 1.21, 1.21, 12.0, 5.7, 3.0, 0.38},
+    {32, 256, 0, 0.85, 0.30, 1.0, 6.3, 3.0, 1.0},     {256, 256, 0, 1.33, 1.33, 4.4, 9.7, 3.7, 0.70},
+    {32, 256, 0, 1.00, 0.40, 2.0, 5.6, 3.0, 1.0},
 };
 
 // The index of the cheapest candidate, -1 where none fits a dispatch.
-inline int pick_deq(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N, int64_t batch, bool ring_ok)
+inline int pick_deq(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N, int64_t batch, bool ring_ok, int64_t cus)
 {
     const double units = (double)((K + 127) / 128);
     int64_t mt[4] = {0, 0, 0, 0}, used = 0, prev = 0, max_rows = 0;  // row tiles of 32, 64, 128 and 256 rows
@@ -136,18 +145,22 @@ inline int pick_deq(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t 
         prev = gl[g];
     }
     const double bytes = (double)batch * ((double)used * K * N + (double)M * (K + 2 * N));
+    const double valid = (double)mt[0] / (8.0 * (double)mt[3]);  // of the 256-row tiles' fragments
+    // the kernel that the call takes without a tile
+    const int untiled = max_rows <= 16               ? DEQ_SKINNY
+                        : max_rows <= kSkinnyMaxRows ? DEQ_SKINNY2
+                        : ring_ok && batch == 1      ? DEQ_RING
+                                                     : DEQ_LDS;
     double best_t = 0;
     int best = -1;
     for (int i = 0; i < (int)(sizeof(kDeqCand) / sizeof(kDeqCand[0])); ++i) {
         const DeqCand& c = kDeqCand[i];
-        if (i == DEQ_SKINNY && max_rows > kSkinnyMaxRows) continue;
-        if (i == DEQ_RING && !ring_ok) continue;
+        if (i >= DEQ_RING && i != untiled) continue;
         int64_t tiles = mt[c.bm == 32 ? 0 : c.bm == 64 ? 1 : c.bm == 128 ? 2 : 3] * ((N + c.bn - 1) / c.bn);
         if (!grid_fits(tiles, c.threads)) continue;
         tiles *= batch;
-        // the ring core's epilogue leaves out 32-row fragments without valid rows
-        const double o = i == DEQ_RING ? 2.0 + 10.0 * (double)mt[0] / (8.0 * (double)mt[3]) : c.o;
-        const double run = tile_rounds_us(tiles, units, c.p, c.r, o);
+        const double k = c.bm == 256 ? c.e + (1.0 - c.e) * valid : 1.0, o = c.bm == 256 ? c.o * (0.2 + 0.8 * valid) : c.o;
+        const double run = tile_rounds_us(tiles, units, c.p * k, c.r * k, o, cus);
         const double mem = bytes / (c.bw * 1e6);
         const double t = c.f + std::sqrt(run * run + mem * mem);
         if (best < 0 || t < best_t) {
@@ -184,7 +197,7 @@ inline constexpr GmmCand kGmmCand[] = {
 };
 
 // The index of the cheapest tile, -1 where none fits a dispatch.
-inline int pick_gmm(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N)
+inline int pick_gmm(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N, int64_t cus)
 {
     const double units = (double)((K + 63) / 64);
     int64_t mt[4] = {0, 0, 0, 0}, used = 0, prev = 0;  // row tiles of 32, 64, 128 and 256 rows
@@ -201,7 +214,7 @@ inline int pick_gmm(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t 
         const GmmCand& c = kGmmCand[i];
         const int64_t tiles = mt[c.bm == 32 ? 0 : c.bm == 64 ? 1 : c.bm == 128 ? 2 : 3] * ((N + c.bn - 1) / c.bn);
         if (!grid_fits(tiles, c.threads)) continue;
-        const double run = tile_rounds_us(tiles, units, c.p, c.r, c.o);
+        const double run = tile_rounds_us(tiles, units, c.p, c.r, c.o, cus);
         const double mem = bytes / (c.bw * 1e6);
         const double t = run * run * run * run + mem * mem * mem * mem;
         if (best < 0 || t < best_t) {

@@ -58,9 +58,9 @@ static GmsqWorkspace gmsq_workspace(int64_t M, int64_t N, int64_t E)
     return w;
 }
 
-// Compute units of the current device (cached per device): the persistent fused kernel keeps one
+// Compute units of the current device: the persistent fused kernel keeps one
 // workgroup per CU.
-static int device_cus()
+int device_cus()
 {
     static int cus[64] = {0};
     int dev = 0;
@@ -139,7 +139,7 @@ static void launch_gemm(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch
         int pick = -1;
         if (tile_ok && g_overrides.gmm_tile > 0 && g_overrides.gmm_tile <= 5) pick = g_overrides.gmm_tile - 1;  // test hook
         else if (tile_ok && g_overrides.persistent_grid == 0)
-            pick = pick_deq(gl, E, a.M, a.K, a.N, batch, a.K >= 4 * PfCfg::BK || batch > 1);
+            pick = pick_deq(gl, E, a.M, a.K, a.N, batch, a.K >= 4 * PfCfg::BK, rule_cus());
         // otherwise the skinny kernel or the 256 x 256 cores below
         if (launch_deq_tile(pick, a, gl, E, batch, st)) return;
     }

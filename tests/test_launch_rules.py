@@ -45,6 +45,7 @@ def test_dqsq_grid(rules, threads):
 # tile numbers of the rules: (rows, columns, threads)
 DEQ_TILES = [(32, 64, 256), (64, 128, 256), (64, 256, 256), (128, 128, 512), (128, 256, 512)]
 GMM_TILES = DEQ_TILES + [(256, 256, 512)]
+RING, SKINNY, LDS = 5, 6, 7  # the other kernels of the int8 rule
 
 
 def _one_group(M):
@@ -103,3 +104,24 @@ def test_gmsq_skip_rule(rules, counts, skips):
 ])
 def test_ring_skip_rule(rules, counts, skips):
     assert bool(rules.rule_ring_skips_empty(_gl(counts), len(counts))) is skips
+
+
+@pytest.mark.parametrize("counts,K,N,batch,kernel", [
+    # wide products of partly filled rounds, and groups of about a tile: the ring core
+    ([1614], 3648, 12288, 1, RING), ([3647], 8640, 4928, 1, RING), ([217] * 16, 3392, 5056, 1, RING),
+    # short K and small batches of more than 32 rows: the 8-wave 256 x 256 kernel, not the ring's constants
+    ([11288], 208, 1088, 1, LDS), ([1862], 96, 6976, 1, LDS), ([94], 832, 1280, 32, LDS), ([1362], 960, 1344, 4, LDS),
+    # small products: tiles that fill the chip; few rows of many experts: the streaming kernel
+    ([24], 7168, 4096, 1, 0), ([300], 7168, 4096, 1, 1), ([8] * 256, 2048, 7168, 1, SKINNY),
+])
+def test_dequant_kernel_choice(rules, counts, K, N, batch, kernel):
+    assert rules.rule_pick_deq(_gl(counts), len(counts), sum(counts), K, N, batch, K >= 256) == kernel
+
+
+@pytest.mark.parametrize("rows", [1, 16, 32])
+@pytest.mark.parametrize("batch", [1, 4])
+def test_dequant_choice_of_few_rows(rules, rows, batch):
+    """Calls whose groups have at most 32 rows have no 256 x 256 kernel: the rule offers none."""
+    for K in (16, 256, 7168):
+        for N in (16, 1024, 16384):
+            assert rules.rule_pick_deq(_gl([rows]), 1, rows, K, N, batch, K >= 256) not in (RING, LDS)
