@@ -5,8 +5,8 @@
 // 116-183; op_kernel/grouped_matmul_kernel.cpp:15-17, 111-150).
 //
 // 16-bit inputs run on v_mfma_f32_32x32x16_{f16,bf16} through the tiles of gemm_tile.hpp (32 x 64 to
-// 256 x 256, chosen by pick_gmm), fp32 accumulation, the bias added in fp32, one
-// round-to-nearest-even narrowing.  Rows or outputs past 32-bit offsets and outputs off 16-byte
+// 256 x 256, chosen by pick_gmm; the 256 x 256 tile of a [N][K] weight with long K is gmm_nk_kernel),
+// fp32 accumulation, the bias added in fp32, one round-to-nearest-even narrowing.  Rows or outputs past 32-bit offsets and outputs off 16-byte
 // alignment take a 128 x 128 register-staged kernel.  fp32 inputs and shapes off the vector path
 // (K or N not a multiple of 8, misaligned operands, 32-bit offsets exceeded) take a plain fp32 loop.
 #include <cstdlib>
@@ -257,6 +257,141 @@ struct GmmTileEpi {
     }
 };
 
+// The 256 x 256 tile for [N][K] weights and long K: 8 waves (4 x 2) of 64 x 128, both operands in 64-deep
+// stages (128 bytes of every row, the tile rows' and the output columns' alike), two stages in LDS, one in
+// flight while the other is multiplied.  tile_gemm_kernel's 256 x 256 tile keeps four stages of 64 bytes:
+// for a [N][K] weight each of its fetches is half of a 128-byte line, and from K of about 1100 on the
+// whole lines of this kernel gain more than the deeper ring (64 x 4672 x 3648, 166 rows per expert:
+// 562 against 613 us; 16 x 1536 x 2944: 50 against 56; 64 x 4096 x 4096, 128 rows: 537 against 531; K 1024:
+// 35 against 32).  Products are summed in the order of that tile (k ascending, one MFMA chain per
+// output), so the two give the same bits.  Chunks past K or N point outside their buffer resource and
+// read zeros.
+constexpr int GL_BM = 256, GL_BN = 256, GL_BK = 64, GL_WN = 2, GL_NT = 512;  // 4 x 2 waves
+constexpr int GL_ROWB = GL_BK * 2;           // bytes per row and stage
+constexpr int GL_A_BYTES = GL_BM * GL_ROWB;  // 32 KB
+constexpr int GL_STAGE = GL_A_BYTES + GL_BN * GL_ROWB;
+constexpr int GL_ISSUE = GL_STAGE / 16 / GL_NT;  // DMAs per thread per stage (8)
+
+template <bool BF16>
+__global__ __launch_bounds__(GL_NT, 1) void gmm_nk_kernel(const GmmFArgs a)
+{
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    constexpr int GROUP_M = 4;
+    const int pid = blockIdx.x;
+    const int T_m = a.gt.total_mtiles, T_n = a.ntiles;
+    const int per_group = GROUP_M * T_n;
+    const int first_m = (pid / per_group) * GROUP_M;
+    const int gsz = (T_m - first_m) < GROUP_M ? (T_m - first_m) : GROUP_M;
+    const int mt = first_m + (pid % per_group) % gsz;
+    const int nt = (pid % per_group) / gsz;
+    const int g = group_of_tile(a.gt, mt);
+    const int rs = g ? a.gt.row_end[g - 1] : 0;
+    const int m0 = rs + (mt - a.gt.tile_start[g]) * GL_BM;
+    const int vrows = a.gt.row_end[g] - m0;
+    const int n0 = nt * GL_BN;
+    const int64_t K = a.K, N = a.N;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / GL_WN, wn = wave % GL_WN;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(CB_LDS uint8_t*)smem;
+
+    const __amdgpu_buffer_rsrc_t ares = make_rsrc((const uint16_t*)a.x + (int64_t)m0 * K,
+                                                     (uint32_t)((vrows < GL_BM ? vrows : GL_BM) * K * 2));
+    const __amdgpu_buffer_rsrc_t bres = make_rsrc((const uint16_t*)a.w + (int64_t)g * K * N, (uint32_t)(K * N * 2));
+    // per DMA i (lane-linear 16-byte chunks of the stage): its k, and the byte offsets at k = 0
+    int kq[4];
+    uint32_t aoff[4], boff[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int cid = (i * 8 + wave) * 64 + lane;
+        const int row = cid >> 3, q = (cid & 7) ^ a_swizzle<8>(row);
+        kq[i] = q * 8;
+        aoff[i] = row < vrows ? (uint32_t)((row * K + q * 8) * 2) : kOffNone;
+        boff[i] = n0 + row < N ? (uint32_t)(((int64_t)(n0 + row) * K + q * 8) * 2) : kOffNone;
+    }
+    const int nk = (int)((K + GL_BK - 1) / GL_BK);
+    auto issue = [&](int kt) {
+        const uint32_t sa = lds_base + (uint32_t)((kt & 1) * GL_STAGE);
+        const int k0 = kt * GL_BK;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            dma16(ares, aoff[i] != kOffNone && k0 + kq[i] < K ? aoff[i] + (uint32_t)(k0 * 2) : kOffNone,
+                  __builtin_amdgcn_readfirstlane(sa + (uint32_t)((i * 8 + wave) * 1024)));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            dma16(bres, boff[i] != kOffNone && k0 + kq[i] < K ? boff[i] + (uint32_t)(k0 * 2) : kOffNone,
+                  __builtin_amdgcn_readfirstlane(sa + GL_A_BYTES + (uint32_t)((i * 8 + wave) * 1024)));
+    };
+
+    f32x16 acc[2][4];
+#pragma unroll
+    for (int fm = 0; fm < 2; ++fm)
+#pragma unroll
+        for (int fn = 0; fn < 4; ++fn) acc[fm][fn] = f32x16{};
+
+    auto frag = [&](const CB_LDS uint8_t* base, const int r, const int q) {
+        return *(const CB_LDS v4i*)(base + r * GL_ROWB + ((q ^ a_swizzle<8>(r)) << 4));
+    };
+    issue(0);
+    issue(1);
+    for (int kt = 0; kt < nk; ++kt) {
+        wait_vmcnt_barrier<GL_ISSUE>();  // stage kt has landed (stage kt + 1 may stay in flight)
+        const CB_LDS uint8_t* st = (const CB_LDS uint8_t*)smem + (kt & 1) * GL_STAGE;
+#pragma unroll
+        for (int ks = 0; ks < GL_BK / 16; ++ks) {
+            v4i af[2], bf[4];
+            const int q = 2 * ks + (lane >> 5);
+#pragma unroll
+            for (int fm = 0; fm < 2; ++fm) af[fm] = frag(st, wm * 64 + fm * 32 + (lane & 31), q);
+#pragma unroll
+            for (int fn = 0; fn < 4; ++fn) bf[fn] = frag(st + GL_A_BYTES, wn * 128 + fn * 32 + (lane & 31), q);
+#pragma unroll
+            for (int fm = 0; fm < 2; ++fm)
+#pragma unroll
+                for (int fn = 0; fn < 4; ++fn) {
+                    if constexpr (BF16) acc[fm][fn] = TileBF16::mma(af[fm], bf[fn], acc[fm][fn]);
+                    else acc[fm][fn] = TileF16::mma(af[fm], bf[fn], acc[fm][fn]);
+                }
+        }
+        // every wave is done with this buffer before the DMA of stage kt + 2 overwrites it
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        issue(kt + 2);  // past K: fetches nothing
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+    // Epilogue.  32x32 C layout: lane l holds column l % 32, rows 8 (r / 4) + 4 (l / 32) + r % 4.
+    // Rows r and r + 1 of a lane pair (l, l ^ 1) are swapped so that each lane stores two adjacent
+    // columns of one row as one dword: the even lane row r, columns (c, c + 1), the odd lane row
+    // r + 1, columns (c - 1, c).  Rows past the group's end fall outside the resource and are dropped.
+    const __amdgpu_buffer_rsrc_t ores = make_rsrc((uint16_t*)a.y + (int64_t)m0 * N,
+                                                  (uint32_t)((vrows < GL_BM ? vrows : GL_BM) * N * 2));
+    const bool odd = lane & 1;
+    float bv[4];
+    uint32_t coff[4];
+#pragma unroll
+    for (int fn = 0; fn < 4; ++fn) {
+        const int64_t col = n0 + wn * 128 + fn * 32 + (lane & 31);
+        bv[fn] = a.bias_dt ? gf_load(a.bias, a.bias_dt, (int64_t)g * N + (col < N ? col : 0)) : 0.0f;
+        coff[fn] = col < N ? (uint32_t)(col & ~(int64_t)1) * 2u : kOffNone;
+    }
+#pragma unroll
+    for (int fm = 0; fm < 2; ++fm)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+            const int lrow = wm * 64 + fm * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);  // rows lrow, lrow + 1
+            const uint32_t roff = (uint32_t)(lrow + (odd ? 1 : 0)) * (uint32_t)N * 2u;
+#pragma unroll
+            for (int fn = 0; fn < 4; ++fn) {
+                const float v0 = acc[fm][fn][r] + bv[fn], v1 = acc[fm][fn][r + 1] + bv[fn];
+                const uint32_t p = BF16 ? pack_bf16x2(v0, v1) : pack_f16x2(v0, v1);
+                // partner lane's pair (quad_perm [1, 0, 3, 2])
+                const uint32_t q = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p, 0xB1, 0xF, 0xF, false);
+                const uint32_t w = odd ? ((q >> 16) | (p & 0xffff0000u)) : ((p & 0xffffu) | (q << 16));
+                __builtin_amdgcn_raw_buffer_store_b32(w, ores, coff[fn] == kOffNone ? kOffNone : roff + coff[fn], 0, 0);
+            }
+        }
+}
+
 // Any dtype and layout: one output element per thread iteration (grid-stride), fp32 accumulation
 // in k order, the bias added in fp32, one narrowing to the output dtype.
 __global__ __launch_bounds__(256) void gmm_generic_kernel(const GmmFArgs a)
@@ -304,6 +439,21 @@ template <class OP, bool BT> using GmmT2 = TileCfg<OP, BT, 2, 4, 1, 2, 2, 1, 3, 
 template <class OP, bool BT> using GmmT3 = TileCfg<OP, BT, 2, 4, 2, 1, 4, 1, 4, 1>;  // 128 x 128, 8 waves
 template <class OP, bool BT> using GmmT4 = TileCfg<OP, BT, 2, 4, 2, 2, 2, 2, 3, 1>;  // 128 x 256, 8 waves
 template <class OP, bool BT> using GmmT5 = TileCfg<OP, BT, 2, 4, 4, 2, 1, 2, 4, 1>;  // 256 x 256, 8 waves
+
+constexpr int64_t kGmmNkMinK = 1152;  // see gmm_nk_kernel
+
+static void launch_gmm_nk(GmmFArgs& a, const int64_t* gl, int64_t E, hipStream_t st)
+{
+    build_group_table(a.gt, gl, E, GL_BM);
+    a.ntiles = (int)((a.N + GL_BN - 1) / GL_BN);
+    const dim3 grid((unsigned)(a.gt.total_mtiles * a.ntiles));
+    auto go = [&](auto kern) {
+        set_dynamic_lds_once((const void*)kern, 2 * GL_STAGE);
+        hipLaunchKernelGGL(kern, grid, dim3(GL_NT), 2 * GL_STAGE, st, a);
+    };
+    if (a.x_dt == CB_DT_BFLOAT16) go(gmm_nk_kernel<true>);
+    else go(gmm_nk_kernel<false>);
+}
 
 }  // namespace cb
 
@@ -359,7 +509,10 @@ extern "C" int cb_grouped_matmul(const void* x, const void* weight, const void* 
             case 2: launch_gmm_tile<GmmT2>(a, group_list, E, st); return check_launch();
             case 3: launch_gmm_tile<GmmT3>(a, group_list, E, st); return check_launch();
             case 4: launch_gmm_tile<GmmT4>(a, group_list, E, st); return check_launch();
-            case 5: launch_gmm_tile<GmmT5>(a, group_list, E, st); return check_launch();
+            case 5:
+                if (a.trans && K >= kGmmNkMinK) launch_gmm_nk(a, group_list, E, st);
+                else launch_gmm_tile<GmmT5>(a, group_list, E, st);
+                return check_launch();
             default: break;
         }
         build_group_table(a.gt, group_list, E, 128);

@@ -173,27 +173,31 @@ inline int pick_deq(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t 
 
 // ---- the 16-bit GroupedMatmul's choice of tile --------------------------------------------------
 // Estimated time of each tile over the call, in the terms of the int8 rule (tile_rounds_us, units of 128
-// bytes of K), combined with the bytes at
-// bw TB/s; the least is taken.  The choice does not look at the weight layout, so that [K][N] and
-// [N][K] storage of the same weights are summed in the same order and agree bit for bit.  Measured
-// us, 64 experts of 4096 x 4096 bf16, [K][N] / [N][K] weights (first: the 256 x 256 double-buffered
-// kernel these replace):
+// bytes of K), combined with the bytes at bw TB/s as the root of the sum of fourth powers (squares put calls
+// near the weight stream's time a tile too low); the least is taken.  The choice does not look at the
+// weight layout, so that [K][N] and [N][K] storage of the same weights are summed in the same order and
+// agree bit for bit.  The constants are fitted to 500 calls (8 to 16384 rows, K and N 256 to 5120, 1 to 64
+// groups, both layouts) on which every tile was timed: the choice is 0.8% off the fastest on average.
+// Measured us, 64 experts of 4096 x 4096 bf16, [K][N] / [N][K] weights, groups drawn unevenly (first: the
+// 256 x 256 double-buffered kernel for every call):
 //   rows per expert     8          24         64         128        256         512
-//   (replaced)       479 / 510  484 / 527  514 / 538  544 / 566  871 / 862  1377 / 1352
-//   32 x 64          377 / 362  419 / 389  583 / 575  855 / 866    -           -
-//   64 x 128         374 / 363  388 / 372  467 / 443  601 / 605  936 / 946     -
-//   64 x 256         346 / 375  354 / 388  444 / 494  540 / 635  870 / 1017    -
-//   128 x 128        402 / 384  409 / 395  437 / 414  554 / 549  845 / 837  1430 / 1401
-//   128 x 256        355 / 372     -       384 / 394  495 / 490  750 / 764  1234 / 1226
-//   256 x 256        409 / 425     -       457 / 485  487 / 544  801 / 875  1241 / 1323
+//   (256 x 256 only) 457 / 493  470 / 498  475 / 517  513 / 537  854 / 793  1332 / 1312
+//   32 x 64          363 / 349  384 / 365  576 / 584  881 / 877    -           -
+//   64 x 128         360 / 349  376 / 361  461 / 451  606 / 592  921 / 927  1651 / 1714
+//   64 x 256         334 / 362  342 / 375  429 / 498  556 / 633  858 / 994  1513 / 1872
+//   128 x 128        392 / 367  403 / 377  429 / 400  566 / 547  837 / 819  1430 / 1429
+//   128 x 256        354 / 359  360 / 366  373 / 383  524 / 487  752 / 724  1246 / 1240
+//   256 x 256        418 / 493  425 / 498  443 / 517  480 / 537  807 / 793  1177 / 1312
+// With 64 rows in every group 64 x 256 takes 361 / 398 and 128 x 256 376 / 384; with 128 rows 491 / 544 and
+// 397 / 410; with 256 rows 128 x 256 takes 645 / 632 and 256 x 256 562 / 603.
 // 8 experts of 2048 x 1536, 8 rows each: 53 -> 13.6 (32 x 64); 1024 rows each: 69 -> 62 (256 x 256).
 struct GmmCand {
     int bm, bn, threads;
     double p, r, o, bw;
 };
 inline constexpr GmmCand kGmmCand[] = {
-    {32, 64, 256, 0.30, 0.152, 1.5, 6.0},  {64, 128, 256, 0.36, 0.34, 2.7, 6.0}, {64, 256, 256, 0.58, 0.66, 5.0, 6.2},
-    {128, 128, 512, 0.42, 0.51, 6.8, 6.2}, {128, 256, 512, 0.90, 0.92, 9.0, 6.2}, {256, 256, 512, 1.30, 1.75, 8.0, 6.2},
+    {32, 64, 256, 0.15, 0.15, 1.8, 6.1},   {64, 128, 256, 0.36, 0.30, 4.7, 6.0},  {64, 256, 256, 0.79, 0.79, 4.8, 6.3},
+    {128, 128, 512, 0.24, 0.46, 7.9, 5.9}, {128, 256, 512, 0.36, 0.82, 10.1, 6.3}, {256, 256, 512, 0.66, 1.55, 10.2, 11.7},
 };
 
 // The index of the cheapest tile, -1 where none fits a dispatch.

@@ -99,6 +99,23 @@ def test_tile_grouped_matmul(cb, orc, overrides, t, counts, K, N, dtype):
     gmm._check(y, ref, dtype, x.float(), w.float(), ends, False)
 
 
+@pytest.mark.parametrize("counts,K,N", [([1, 0, 33, 300], 1152, 264), ([256, 257, 31], 1208, 72), ([513], 1600, 776)])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("bias", ["f32", None])
+def test_grouped_matmul_long_k_layouts(cb, orc, overrides, counts, K, N, dtype, bias):
+    """From K of 1152 on the 256 x 256 tile of a [N][K] weight is a kernel of its own: the oracle's result, and the
+    bits of the [K][N] kernel."""
+    overrides(gmm_tile=6)
+    x, w, b, ends = gmm._inputs(counts, K, N, dtype, False, bias, K + N)
+    args = dict(bias=None if b is None else b.to(DEV), split_item=2)
+    y = cb.grouped_matmul(x.to(DEV), w.to(DEV), ends, **args)[0]
+    yt = cb.grouped_matmul(x.to(DEV), w.transpose(1, 2).contiguous().to(DEV), ends, transpose_weight=True, **args)[0]
+    assert torch.equal(y.view(torch.int16), yt.view(torch.int16))
+    ref = orc.grouped_matmul(gmm.host(x, dtype), gmm.host(w, dtype), ends, None if b is None else b.numpy(), dtype=dtype,
+                             bias_dtype=bias or "f32")
+    gmm._check(yt, ref, dtype, x.float(), w.float(), ends, False)
+
+
 @pytest.mark.parametrize("off", [1, 2, 4])  # elements: y at 2, 4 and 8 bytes past a 16-byte boundary
 def test_grouped_matmul_unaligned_output(cb, off):
     """An output off 16-byte alignment (possible through the C ABI) takes the kernel with single-value

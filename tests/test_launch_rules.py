@@ -125,3 +125,11 @@ def test_dequant_choice_of_few_rows(rules, rows, batch):
     for K in (16, 256, 7168):
         for N in (16, 1024, 16384):
             assert rules.rule_pick_deq(_gl([rows]), 1, rows, K, N, batch, K >= 256) not in (RING, LDS)
+
+
+@pytest.mark.parametrize("counts,K,N,tile", [
+    ([156] * 32, 2496, 4352, 5), ([175] * 8, 1984, 4416, 5), ([1687, 1688], 4544, 3776, 5),  # uneven rounds, long K
+    ([8] * 64, 4096, 4096, 2), ([256] * 64, 4096, 4096, 5), ([64] * 64, 4096, 4096, 2),
+])
+def test_grouped_matmul_tile_choice(rules, counts, K, N, tile):
+    assert rules.rule_pick_gmm(_gl(counts), len(counts), sum(counts), K, N) == tile
