@@ -26,6 +26,12 @@ inline int64_t dqsq_blocks(int64_t M, int64_t threads)
     return want < most ? want : most;
 }
 
+// Workgroups of the decode-shaped GroupedMatmulSwigluQuant, which draw ntl tiles for each group with rows:
+// one per CU (cus), at most ntl for every group, with rows or without.  A grid of only as many
+// workgroups as there are tiles was slower: 22 of 256 experts (198 tiles of 5568 x 2176) take 72 to 105 us
+// from 256 workgroups, 108 from 198.
+inline int64_t gmsq_decode_grid(int64_t groups, int64_t ntl, int64_t cus) { return groups * ntl < cus ? groups * ntl : cus; }
+
 // How groups fill 256-row tiles.
 struct TileFill {
     int64_t frags = 0, tiles = 0, max_rows = 0;  // 32-row fragments with valid rows, 256-row tiles

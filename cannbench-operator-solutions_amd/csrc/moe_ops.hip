@@ -255,9 +255,9 @@ static int launch_gmsq_decode(GemmArgs& a, const int64_t* group_list, int64_t E,
         resident = 0;
     build_group_table(a.gt, group_list, E, 16 * kDecRB);
     const int64_t tiles = (int64_t)a.gt.total_mtiles * ntl;
-    int grid = (resident < 1 ? resident : 1) * cus;
+    int grid = (int)gmsq_decode_grid(E, ntl, (resident < 1 ? resident : 1) * cus);
     if (g_overrides.persistent_grid > 0 && resident >= 1) grid = g_overrides.persistent_grid;  // test hook
-    if (grid > tiles) grid = (int)tiles;
+    if (grid > E * ntl) grid = (int)(E * ntl);
     if (grid < 1) return -1;
     a.ntiles = ntl;
     clear_ws(tiles);

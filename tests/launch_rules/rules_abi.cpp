@@ -13,5 +13,6 @@ int rule_gmsq_skips_empty(const int64_t* gl, int64_t E, int64_t ntl, int64_t gri
 {
     return cb::gmsq_skips_empty(gl, E, ntl, grid);
 }
+int64_t rule_gmsq_decode_grid(int64_t groups, int64_t ntl, int64_t cus) { return cb::gmsq_decode_grid(groups, ntl, cus); }
 int rule_ring_skips_empty(const int64_t* gl, int64_t E) { return cb::ring_skips_empty(gl, E); }
 }

@@ -27,6 +27,8 @@ def rules(tmp_path_factory):
     lib.rule_pick_gmm.argtypes = [gl, i64, i64, i64, i64]
     lib.rule_gmsq_skips_empty.argtypes = [gl, i64, i64, i64]
     lib.rule_ring_skips_empty.argtypes = [gl, i64]
+    lib.rule_gmsq_decode_grid.argtypes = [i64, i64, i64]
+    lib.rule_gmsq_decode_grid.restype = i64
     return lib
 
 
@@ -133,3 +135,12 @@ def test_dequant_choice_of_few_rows(rules, rows, batch):
 ])
 def test_grouped_matmul_tile_choice(rules, counts, K, N, tile):
     assert rules.rule_pick_gmm(_gl(counts), len(counts), sum(counts), K, N) == tile
+
+
+def test_gmsq_decode_grid(rules):
+    """One workgroup per CU; fewer only where the call has fewer column tiles in all its groups, empty ones
+    included."""
+    assert rules.rule_gmsq_decode_grid(256, 9, 256) == 256
+    assert rules.rule_gmsq_decode_grid(8, 5, 256) == 40
+    assert rules.rule_gmsq_decode_grid(1, 1, 256) == 1
+    assert rules.rule_gmsq_decode_grid(256, 16, 0) == 0  # the kernel cannot be resident
