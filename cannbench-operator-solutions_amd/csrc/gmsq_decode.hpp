@@ -18,7 +18,10 @@
 
 namespace cb {
 
-constexpr int kDecRB = 2;  // 16-row blocks per tile (3: 48 rows, level with the prefill kernel; 4 spills)
+// 16-row blocks per tile: groups of this kernel have one row tile each.  (3, for groups of up to 48 rows,
+// took 1201 and 1242 us where the prefill kernel then took 1325 and 1337 (256 experts of 7168 x 4096, up to 46
+// rows); that kernel has left out empty fragments since, 1282 at 47 rows each.  4 spills.)
+constexpr int kDecRB = 2;
 
 // The product, SwiGLU and row maxima of one tile: RB 16-row blocks of expert g from row r0 on (rows
 // below r1) x 128 act columns.  Lane (q, c), c < 8, ends with act[rb][j] = act of row r0 + 16 rb +
@@ -225,9 +228,10 @@ __device__ __forceinline__ void decode_finish(const GemmArgs& a, const int mt, c
     }
 }
 
-// Persistent decode kernel with dynamic tile order.  The tiles (expert g, 128-act-column tile ct)
-// are numbered in expert order, t = g * ntiles + ct, and the workgroups draw them with one atomic
-// ticket, so a faster CU simply takes more tiles.  (Measured: one list in expert order beats 8
+// Persistent decode kernel with dynamic tile order.  The tiles (row tile mt, 128-act-column tile ct)
+// are numbered in expert order, t = mt * ntiles + ct, where mt counts the experts that have rows (looked
+// up in the group table: searching it cost tiles of few rows 4%, 8 experts of 6400 x 640 with 3 rows each
+// 61 against 59 us), and the workgroups draw them with one atomic ticket, so a faster CU simply takes more tiles.  (Measured: one list in expert order beats 8
 // per-XCD lists, each holding a quarter of the experts and half of the columns.)  An expert's
 // column tiles are drawn together, so they finish together: each tile publishes its row maxima
 // into the self-validating slots as soon as its product is done, and its requant is deferred until
@@ -255,17 +259,15 @@ __global__ __launch_bounds__(256, 1) void gmsq_decode_kernel(const GemmArgs a)
     if (threadIdx.x == 0) next_t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     int t = (int)next_t;
-    __syncthreads();  // every wave has read next_t before thread 0 rewrites it (an empty expert's
-                      // iteration has no barrier of its own)
+    __syncthreads();  // every wave has read next_t before thread 0 rewrites it
     int pm = -1, pct = 0, pr0 = 0, pr1 = 0;  // the deferred tile
     while (t < count) {
         // draw the next ticket now; its result is needed only after this tile
         u32 nt_pending = 0;
         if (threadIdx.x == 0) nt_pending = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const int mt = t / ntl, ct = t % ntl;
-        const int g = group_of_tile(a.gt, mt);
-        const int r0 = (g ? a.gt.row_end[g - 1] : 0) + (mt - a.gt.tile_start[g]) * 16 * kDecRB;
-        const int r1 = r0 + 16 * kDecRB < a.gt.row_end[g] ? r0 + 16 * kDecRB : a.gt.row_end[g];
+        const int g = a.gt.tile_start[mt];  // build_decode_table
+        const int r0 = g ? a.gt.row_end[g - 1] : 0, r1 = a.gt.row_end[g];
         {
             float act[kDecRB][16];
             u32 rmax[kDecRB];
@@ -323,9 +325,8 @@ __global__ __launch_bounds__(256, 1) void gmsq_decode_fixup_kernel(const GemmArg
         if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(a.epi.redo + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
             continue;
         const int mt = t / a.ntiles, ct = t % a.ntiles;
-        const int g = group_of_tile(a.gt, mt);
-        const int r0 = (g ? a.gt.row_end[g - 1] : 0) + (mt - a.gt.tile_start[g]) * 16 * kDecRB;
-        const int r1 = r0 + 16 * kDecRB < a.gt.row_end[g] ? r0 + 16 * kDecRB : a.gt.row_end[g];
+        const int g = a.gt.tile_start[mt];  // build_decode_table
+        const int r0 = g ? a.gt.row_end[g - 1] : 0, r1 = a.gt.row_end[g];
         float act[kDecRB][16];
         u32 rmax[kDecRB];
         decode_tile_act(a, g, ct, r0, r1, red, act, rmax);

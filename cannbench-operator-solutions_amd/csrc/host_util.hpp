@@ -19,7 +19,8 @@ inline bool offsets32_ok(int64_t K, int64_t N) { return K * N < (1LL << 31); }
 
 // Cumsum group boundaries plus the prefix of M-tiles per group, passed by value to the grouped
 // kernels (no host->device copy, no device allocation).  row_end[g] is the exclusive end row of
-// group g; tile_start[g] is the first M-tile of group g in the launch's tile enumeration.
+// group g; tile_start[g] is the first M-tile of group g in the launch's tile enumeration (the decode kernel has a
+// table of its own, build_decode_table).
 struct GroupTable {
     int32_t n_groups;
     int32_t total_mtiles;
@@ -67,6 +68,18 @@ inline void build_group_table(GroupTable& t, const int64_t* gl, int64_t E, int b
     t.tile_start[CB_MAX_EXPERTS] = tiles;
     t.total_mtiles = tiles;
     t.max_rows = mx;
+}
+
+// The table of the decode kernel, whose groups are at most one row tile: tile_start[i] is the group of
+// row tile i (the i-th non-empty group), so a workgroup finds its tile's rows without a search.
+inline void build_decode_table(GroupTable& t, const int64_t* gl, int64_t E)
+{
+    build_group_table(t, gl, E, 32);
+    int32_t tiles = 0, prev = 0;
+    for (int32_t g = 0; g < t.n_groups; ++g) {
+        if (t.row_end[g] > prev) t.tile_start[tiles++] = g;
+        prev = t.row_end[g];
+    }
 }
 
 inline int check_launch()

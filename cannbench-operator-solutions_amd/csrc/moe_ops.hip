@@ -253,7 +253,7 @@ static int launch_gmsq_decode(GemmArgs& a, const int64_t* group_list, int64_t E,
     int resident = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, (const void*)gmsq_decode_kernel, 256, 0) != hipSuccess)
         resident = 0;
-    build_group_table(a.gt, group_list, E, 16 * kDecRB);
+    build_decode_table(a.gt, group_list, E);
     const int64_t tiles = (int64_t)a.gt.total_mtiles * ntl;
     int grid = (int)gmsq_decode_grid(E, ntl, (resident < 1 ? resident : 1) * cus);
     if (g_overrides.persistent_grid > 0 && resident >= 1) grid = g_overrides.persistent_grid;  // test hook
