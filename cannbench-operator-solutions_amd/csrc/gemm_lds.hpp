@@ -64,14 +64,10 @@ struct LdsCfg {
     // [256][128]) with a 16-byte row pad that keeps rows 4 apart off the same banks
     static constexpr int EPI_PITCH = 528;
     static constexpr int EPI_BYTES = BM * EPI_PITCH;
-    // the tile's per-row activation scales (SwiGLU epilogues), after the ring / staging area
-    // and the column scales: one slot of BM + BN floats
+    // the tile's row and column scales (dequant epilogue), after the ring / staging area
     static constexpr int XS_OFF = STAGES * STAGE > EPI_BYTES ? STAGES * STAGE : EPI_BYTES;
-    static constexpr int XS_SLOT = (BM + BN) * 4;
-    static constexpr int LDS_BYTES = XS_OFF + XS_SLOT;
-    // persistent dequant / int32 kernel: the ring, then two scale slots (alternate tiles)
-    static constexpr int CONT_XS_OFF = STAGES * STAGE;
-    static constexpr int CONT_LDS_BYTES = CONT_XS_OFF + 2 * XS_SLOT;
+    static constexpr int LDS_BYTES = XS_OFF + (BM + BN) * 4;
+    static constexpr int CONT_LDS_BYTES = STAGES * STAGE;  // the persistent int32 kernel: the ring alone
     static constexpr int A_ISSUE = A_BYTES / 16 / NT;  // DMA instructions per thread per stage
     static constexpr int B_ISSUE = B_BYTES / 16 / NT;
     static constexpr int ISSUE = A_ISSUE + B_ISSUE;
@@ -206,9 +202,9 @@ template <int EPI, int WM, int WN, int STAGES, int BKT>
 using TileDmaOf = TileDma<LdsCfg<WM, WN, STAGES, BKT>, false>;
 
 // One 256 x 256 output tile (row tile mt, column tile nt, batch b).  Called once per workgroup by
-// lds_gemm_kernel and in a loop by the persistent kernels.
+// lds_gemm_kernel and in a loop by the persistent kernel.
 //
-// CONT (continuous stage stream, persistent dequant / int32 kernel): the tile's first STAGES stages
+// CONT (continuous stage stream, the persistent int32 kernel): the tile's first STAGES stages
 // were already issued by the previous tile (or the kernel's prologue) from the plan `cur` into ring
 // slots sbase, sbase + 1, ...; the last STAGES iterations of this tile issue the first stages of
 // the plan `nxt`.  The epilogue then writes from registers and leaves the LDS ring to those DMAs.
@@ -217,7 +213,7 @@ __device__ __forceinline__ void lds_gemm_tile(const GemmArgs& a, const int mt, c
                                               uint8_t* smem,
                                               const TileDmaOf<EPI, WM, WN, STAGES, BKT>* cur = nullptr,
                                               const TileDmaOf<EPI, WM, WN, STAGES, BKT>* nxt = nullptr,
-                                              const int sbase = 0, const int xs_slot = 0)
+                                              const int sbase = 0)
 {
     using C = LdsCfg<WM, WN, STAGES, BKT>;
     constexpr int KS = C::KS, ACH = C::ACH;
@@ -235,7 +231,7 @@ __device__ __forceinline__ void lds_gemm_tile(const GemmArgs& a, const int mt, c
     const int m0 = rs + (mt - a.gt.tile_start[g]) * BM;
     const int vrows = r1 - m0;  // valid rows of this tile (>= 1)
 
-    static_assert(EPI == EPI_DEQUANT || EPI == EPI_I32, "dequant / int32 epilogues only");
+    static_assert(EPI == EPI_I32 || (EPI == EPI_DEQUANT && !CONT), "dequant / int32 epilogues only");
     TileDma<C, false> dma;
     if constexpr (CONT) dma = *cur;
     else dma.init(a, mt, nt, b, wave, lane);
@@ -327,18 +323,12 @@ __device__ __forceinline__ void lds_gemm_tile(const GemmArgs& a, const int mt, c
         const uint16_t b16 = __builtin_amdgcn_raw_buffer_load_b16(s16, (uint32_t)(si * 2), 0, 0);
         cs_pre = e.scale_bf16 ? bf16_to_f32(b16) : f32;
     }
-    CB_LDS float* xs_lds =
-        (CB_LDS float*)((CB_LDS uint8_t*)smem + (CONT ? C::CONT_XS_OFF + xs_slot * C::XS_SLOT : C::XS_OFF));
+    CB_LDS float* xs_lds = (CB_LDS float*)((CB_LDS uint8_t*)smem + C::XS_OFF);
     CB_LDS float* cs_lds = xs_lds + BM;
     auto publish_scales = [&]() {
         if (tid < BM) xs_lds[tid] = xs_pre;
         if (tid < BN) cs_lds[tid] = cs_pre;
     };
-    if constexpr (CONT && EPI == EPI_DEQUANT) {
-        // no barrier of its own in this epilogue: the K loop's barriers publish the slot (the
-        // previous tile read the other one)
-        publish_scales();
-    }
 
     // Software pipeline per stage kt (fragments of half-stage ks = 0 already in registers):
     //   read ks = 1 fragments | MFMAs on ks = 0 | barrier for stage kt + 1, refill the buffer
@@ -429,81 +419,21 @@ __device__ __forceinline__ void lds_gemm_tile(const GemmArgs& a, const int mt, c
         // no branch whose join would make the compiler wait for the stores issued before it.
         // Column offsets of fragment fn: col0 + 32 fn, outside the resource past N.
         const int64_t col0 = (int64_t)nt * BN + wn * TN + (lane & 31);
-        if constexpr (EPI == EPI_I32) {
-            const __amdgpu_buffer_rsrc_t ores =
-                make_rsrc((int32_t*)e.out + b * e.out_bstride + (int64_t)m0 * N, (uint32_t)((vrows < BM ? vrows : BM) * N * 4));
-            uint32_t coff[FN];
+        const __amdgpu_buffer_rsrc_t ores =
+            make_rsrc((int32_t*)e.out + b * e.out_bstride + (int64_t)m0 * N, (uint32_t)((vrows < BM ? vrows : BM) * N * 4));
+        uint32_t coff[FN];
 #pragma unroll
-            for (int fn = 0; fn < FN; ++fn) coff[fn] = col0 + 32 * fn < N ? (uint32_t)(col0 + 32 * fn) * 4u : 0x80000000u;
+        for (int fn = 0; fn < FN; ++fn) coff[fn] = col0 + 32 * fn < N ? (uint32_t)(col0 + 32 * fn) * 4u : 0x80000000u;
 #pragma unroll
-            for (int fm = 0; fm < FM; ++fm) {
+        for (int fm = 0; fm < FM; ++fm) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int lrow = (WM * fm + wm) * 32 + (r >> 2) * 8 + lr + (r & 3);
-                    const uint32_t roff = (uint32_t)lrow * (uint32_t)N * 4u;
+            for (int r = 0; r < 16; ++r) {
+                const int lrow = (WM * fm + wm) * 32 + (r >> 2) * 8 + lr + (r & 3);
+                const uint32_t roff = (uint32_t)lrow * (uint32_t)N * 4u;
 #pragma unroll
-                    for (int fn = 0; fn < FN; ++fn)
-                        __builtin_amdgcn_raw_buffer_store_b32(acc[fm][fn][r], ores, roff + coff[fn], 0, 0);
-                }
+                for (int fn = 0; fn < FN; ++fn)
+                    __builtin_amdgcn_raw_buffer_store_b32(acc[fm][fn][r], ores, roff + coff[fn], 0, 0);
             }
-        } else {
-            // Rows r and r + 1 of a lane pair (l, l ^ 1) are swapped so that each lane stores two
-            // adjacent columns of one row as one dword: the even lane row r, columns (c, c + 1),
-            // the odd lane row r + 1, columns (c - 1, c).
-            const __amdgpu_buffer_rsrc_t ores =
-                make_rsrc((uint16_t*)e.out + b * e.out_bstride + (int64_t)m0 * N, (uint32_t)((vrows < BM ? vrows : BM) * N * 2));
-            const bool odd = lane & 1;
-            ColDeq cd[FN];
-            uint32_t coff[FN];
-            const bool full_chain = e.has_offset || e.bias_kind != BIAS_NONE;  // uniform
-#pragma unroll
-            for (int fn = 0; fn < FN; ++fn) {
-                const int64_t cc = col0 + 32 * fn;
-                if (full_chain) cd[fn] = col_deq(e, g, b, cc < N ? cc : 0);
-                else cd[fn] = ColDeq{cs_lds[wn * TN + fn * 32 + (lane & 31)], 0.0f, 0.0f};
-                coff[fn] = cc < N ? (uint32_t)(cc & ~(int64_t)1) * 2u : 0x80000000u;
-            }
-            // the row scales come from LDS (fetched under the K loop): no global load between the
-            // stores, whose wait would drain every store issued before it (vmcnt counts stores too)
-            float ptv[FM][16];
-#pragma unroll
-            for (int fm = 0; fm < FM; ++fm)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) ptv[fm][r] = xs_lds[(WM * fm + wm) * 32 + (r >> 2) * 8 + lr + (r & 3)];
-            auto store = [&](auto simple_const) {
-                constexpr bool SIMPLE = decltype(simple_const)::value;
-#pragma unroll
-                for (int fm = 0; fm < FM; ++fm) {
-    #pragma unroll
-                    for (int r = 0; r < 16; r += 2) {
-                        const int lrow = (WM * fm + wm) * 32 + (r >> 2) * 8 + lr + (r & 3);  // rows lrow, lrow + 1
-                        const float pt0 = ptv[fm][r], pt1 = ptv[fm][r + 1];
-                        const uint32_t roff = (uint32_t)(lrow + (odd ? 1 : 0)) * (uint32_t)N * 2u;
-#pragma unroll
-                        for (int fn = 0; fn < FN; ++fn) {
-                            uint32_t h0, h1;
-                            if constexpr (SIMPLE) {
-                                h0 = f32_to_bf16_hw(((float)acc[fm][fn][r] * cd[fn].scale) * pt0);
-                                h1 = f32_to_bf16_hw(((float)acc[fm][fn][r + 1] * cd[fn].scale) * pt1);
-                            } else {
-                                const float v0 = apply_deq(e, cd[fn], acc[fm][fn][r], pt0);
-                                const float v1 = apply_deq(e, cd[fn], acc[fm][fn][r + 1], pt1);
-                                h0 = e.out_bf16 ? f32_to_bf16_hw(v0) : f32_to_f16(v0);
-                                h1 = e.out_bf16 ? f32_to_bf16_hw(v1) : f32_to_f16(v1);
-                            }
-                            const uint32_t p = h0 | (h1 << 16);
-                            // partner lane's pair (quad_perm [1, 0, 3, 2])
-                            const uint32_t q = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p, 0xB1, 0xF, 0xF, false);
-                            const uint32_t w = odd ? ((q >> 16) | (p & 0xffff0000u)) : ((p & 0xffffu) | (q << 16));
-                            __builtin_amdgcn_raw_buffer_store_b32(w, ores, roff + coff[fn], 0, 0);
-                        }
-                    }
-                }
-            };
-            if (!e.has_offset && e.bias_kind == BIAS_NONE && e.out_bf16)
-                store(std::integral_constant<bool, true>());
-            else
-                store(std::integral_constant<bool, false>());
         }
     } else if constexpr (EPI == EPI_I32) {
         int32_t* ob = (int32_t*)e.out + b * e.out_bstride;
@@ -615,11 +545,11 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void lds_gemm_kernel(const GemmArg
     lds_gemm_tile<EPI, WM, WN, STAGES, BKT>(a, mt, nt, blockIdx.y, smem);
 }
 
-// Persistent dequant / int32 GEMM (batch 1): gridDim.x workgroups, one per CU, walk the tiles
+// Persistent int32 GEMM (batch 1): gridDim.x workgroups, one per CU, walk the tiles
 // pid = blockIdx.x, blockIdx.x + gridDim.x, ... of the non-persistent order.  One continuous stage
 // stream per workgroup: a tile's last STAGES iterations DMA the next tile's first stages, so no tile
 // starts with an empty ring, and the register-direct epilogue overlaps those DMAs.
-template <int EPI, int WM, int WN, int STAGES, int BKT>
+template <int WM, int WN, int STAGES, int BKT>
 __global__ __launch_bounds__(64 * WM * WN, 1) void lds_gemm_persistent_kernel(const GemmArgs a)
 {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -629,13 +559,13 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void lds_gemm_persistent_kernel(co
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lds_base = (uint32_t)(uintptr_t)(CB_LDS uint8_t*)smem;
-    TileDmaOf<EPI, WM, WN, STAGES, BKT> cur, nxt;
+    TileDmaOf<EPI_I32, WM, WN, STAGES, BKT> cur, nxt;
     int mt, nt;
     tile_of_pid(a, pid, mt, nt);
     cur.init(a, mt, nt, 0, wave, lane);
 #pragma unroll
     for (int st = 0; st < STAGES; ++st) cur.issue_at(st, st, lds_base, wave);
-    int sbase = 0, xs_slot = 0;
+    int sbase = 0;
     for (;;) {
         const int pn = pid + (int)gridDim.x;
         int mt2 = 0, nt2 = 0;
@@ -645,9 +575,8 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void lds_gemm_persistent_kernel(co
         } else {
             nxt.set_dead(a);
         }
-        lds_gemm_tile<EPI, WM, WN, STAGES, BKT, true>(a, mt, nt, 0, smem, &cur, &nxt, sbase, xs_slot);
+        lds_gemm_tile<EPI_I32, WM, WN, STAGES, BKT, true>(a, mt, nt, 0, smem, &cur, &nxt, sbase);
         if (pn >= total) break;
-        xs_slot ^= 1;
         sbase = (sbase + cur.nk) % STAGES;
         cur = nxt;
         pid = pn;

@@ -181,17 +181,18 @@ static void launch_gemm(GemmArgs& a, const int64_t* gl, int64_t E, int64_t batch
             return;
         }
     }
-    // persistent launch once there are more tiles than workgroups (one continuous DMA stream per
-    // workgroup: a tile's last STAGES iterations issue the next tile's first STAGES stages, so K
-    // must span at least STAGES stages); its register-direct epilogue addresses a tile's rows with
-    // 32-bit offsets
-    if (batch == 1 && pg > 0 && blocks > pg && a.K >= (int64_t)Cfg::STAGES_ * Cfg::BK &&
-        Cfg::BM * Ncols * 4 < 0x7fffffffLL) {
-        auto kern = lds_gemm_persistent_kernel<EPI, kLdsWM, kLdsWN, kLdsStages, kLdsBK>;
-        constexpr int lds = Cfg::CONT_LDS_BYTES;  // the ring and two row-scale slots
-        set_dynamic_lds_once((const void*)kern, lds);
-        hipLaunchKernelGGL(kern, dim3((unsigned)pg), dim3(Cfg::NT), lds, st, a);
-        return;
+    if constexpr (EPI == EPI_I32) {
+        // persistent launch once there are more tiles than workgroups (one continuous DMA stream per
+        // workgroup: a tile's last STAGES iterations issue the next tile's first STAGES stages, so K
+        // must span at least STAGES stages); its register-direct epilogue addresses a tile's rows with
+        // 32-bit offsets.  (A dequant GEMM with such a K runs on the ring core.)
+        if (batch == 1 && pg > 0 && blocks > pg && a.K >= (int64_t)Cfg::STAGES_ * Cfg::BK &&
+            Cfg::BM * Ncols * 4 < 0x7fffffffLL) {
+            auto kern = lds_gemm_persistent_kernel<kLdsWM, kLdsWN, kLdsStages, kLdsBK>;
+            set_dynamic_lds_once((const void*)kern, Cfg::CONT_LDS_BYTES);
+            hipLaunchKernelGGL(kern, dim3((unsigned)pg), dim3(Cfg::NT), Cfg::CONT_LDS_BYTES, st, a);
+            return;
+        }
     }
     auto kern = lds_gemm_kernel<EPI, kLdsWM, kLdsWN, kLdsStages, kLdsBK>;
     set_dynamic_lds_once((const void*)kern, Cfg::LDS_BYTES);
