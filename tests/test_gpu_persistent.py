@@ -1,10 +1,14 @@
-"""GPU parity of the persistent dequant / int32 GEMM (one continuous DMA stage stream per workgroup).
+"""GPU parity of the persistent dequant / int32 GEMM (one continuous DMA stage stream per workgroup) and
+of the 8-wave kernel with one tile per workgroup beside it.
 
-These tests force a small grid with the library's test override, so every workgroup walks many
-tiles (the dequant GEMM on the ring core and the 8-wave int32 GEMM).  Together the cases cover an odd number of K stages (the ring rotates between tiles), both launch orders of the ring core (row tile runs; 4 x 8 tile blocks per XCD), K of
-exactly the ring's depth, K shorter than the ring (launched one tile per workgroup instead), ragged
-and empty groups, partial row and column tiles, every dequant flag, and the last tile's stages that
-fetch nothing.  The bar is the same as the non-persistent path: bit-exact against the oracle.
+Most tests force a small grid with the library's test override, so every workgroup walks many
+tiles (the dequant GEMM on the ring core and the 8-wave int32 GEMM; a forced grid also keeps the
+dequant GEMM from choosing a smaller tile).  Together the cases cover an odd number of K stages (the
+ring rotates between tiles), both launch orders of the ring core (row tile runs; 4 x 8 tile blocks
+per XCD), its epilogue with and without empty fragments, K of exactly the ring's depth, K shorter
+than the ring (the 8-wave kernel, one tile per workgroup), ragged and empty groups, partial row and
+column tiles, every dequant flag, and the last tile's stages that fetch nothing.  The bar is
+bit-exact against the oracle.
 """
 import numpy as np
 import pytest
@@ -46,8 +50,7 @@ GMQ_CASES = [
     # tiles x 8 column tiles per XCD and round), with a partial last band of row tiles
     ([520, 17, 0, 700], 256, 2040),
     ([300, 0, 45, 600, 1, 0, 33, 256, 90], 448, 4096),
-    # N % 8 == 4 with K of at least 4 stages: the ring core's 16-byte stores need N % 8 == 0, so
-    # these take the 8-wave persistent kernel
+    # N off the 16-column vectors: the kernel with one output per thread
     ([300, 0, 45, 600], 384, 772),
 ]
 
@@ -116,8 +119,7 @@ def test_persistent_quant_matmul_flags(cb, orc, small_grid, variant):
 
 @pytest.mark.parametrize("N", [772, 100])
 def test_quant_matmul_n_mod8_4(cb, orc, small_grid, N):
-    """QuantMatmul with N % 8 == 4 and K >= 256 (outside the ring core's 16-byte store gate):
-    bit-exact against the oracle on the kernel these shapes take."""
+    """QuantMatmul with N off the 16-column vectors, which takes the kernel with one output per thread."""
     g = cpu_gen(N)
     M, K = 300, 512
     x1 = rand_i8((M, K), g)
@@ -155,6 +157,48 @@ def test_persistent_default_grid_matches_one_tile_per_workgroup(cb, overrides):
         for r in {s, s + cnt - 1} if cnt else ():
             np.testing.assert_array_equal(cn[r], xn[r] @ wn[e], err_msg=f"group {e} row {r}")
         s += cnt
+
+
+@pytest.mark.parametrize("counts,K,N", [
+    ([600, 13, 0, 700, 256, 640, 1, 550, 900], 256, 4096),  # 304 tiles: the block launch order
+    ([270] * 20, 320, 2000),                                # 320 tiles: runs of row tiles, a full and a light one per group
+])
+def test_ring_on_its_default_grid(cb, overrides, counts, K, N):
+    """The ring core on one workgroup per CU, whatever the rule would choose, against the 8-wave kernel with one
+    tile per workgroup."""
+    g = cpu_gen(K + N)
+    E, M = len(counts), sum(counts)
+    x, w = rand_i8((M, K), g), rand_i8((E, K, N), g)
+    ws = (torch.rand(E, N, generator=g) * 0.009 + 0.001).to(DEV)
+    xs = (torch.rand(M, generator=g) * 0.015 + 0.005).to(DEV)
+    gl = np.cumsum(counts).tolist()
+    overrides(persistent_grid=torch.cuda.get_device_properties(0).multi_processor_count)
+    a = cb.grouped_matmul_quant(x, w, ws, xs, gl)
+    overrides(persistent_grid=-1)
+    b = cb.grouped_matmul_quant(x, w, ws, xs, gl)
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("grid", [-1, 0])  # the 8-wave kernel forced; the rule's choice
+@pytest.mark.parametrize("B,M,K,N", [(3, 40, 256, 96), (2, 300, 272, 528), (4, 1362, 960, 1344)])
+@pytest.mark.parametrize("flags", ["bias", "full"])
+def test_batched_quant_matmul(cb, orc, overrides, grid, B, M, K, N, flags):
+    """Batches of more than 32 rows with a bias per batch, with and without an offset: bit-exact against the
+    oracle, batch by batch."""
+    rng = np.random.default_rng(B + M)
+    x1, x2 = (rng.integers(-127, 128, size=s, dtype=np.int8) for s in ((B, M, K), (B, K, N)))
+    scale = rng.uniform(0.001, 0.01, N).astype(np.float32)
+    bias = rng.integers(-5000, 5000, (B, 1, N), dtype=np.int32) if flags == "bias" else rng.normal(size=(B, 1, N)).astype(np.float32)
+    off = rng.uniform(-1, 1, N).astype(np.float32) if flags == "full" else None
+    pt = rng.uniform(0.005, 0.02, M).astype(np.float32) if flags == "full" else None
+    opt = lambda a: None if a is None else torch.from_numpy(a).to(DEV)
+    overrides(persistent_grid=grid)
+    out = cb.quant_matmul(opt(x1), opt(x2), opt(scale), offset=opt(off), pertoken_scale=opt(pt), bias=opt(bias),
+                          output_dtype="bfloat16")
+    for b in range(B):
+        ref = orc.quant_matmul(x1[b], x2[b], scale, offset=off, pertoken=pt, bias=bias[b, 0],
+                               bias_dtype="i32" if flags == "bias" else "f32", out_dtype="bf16")
+        np.testing.assert_array_equal(bits16(out[b]).reshape(ref.shape), ref, err_msg=f"batch {b}")
 
 
 @pytest.mark.parametrize("counts,K,N", [
