@@ -35,6 +35,7 @@ inline int64_t gmsq_decode_grid(int64_t groups, int64_t ntl, int64_t cus) { retu
 // How groups fill 256-row tiles.
 struct TileFill {
     int64_t frags = 0, tiles = 0, max_rows = 0;  // 32-row fragments with valid rows, 256-row tiles
+    int64_t used = 0, heavy = 0;                 // groups with rows, with more than 256
     bool mostly_empty() const { return 2 * frags < 9 * tiles; }  // under 9 of 16 fragments
 };
 
@@ -46,6 +47,8 @@ inline TileFill tile_fill(const int64_t* gl, int64_t E)
         const int64_t rows = gl[g] - prev;
         f.frags += (rows + 31) / 32;
         f.tiles += (rows + 255) / 256;
+        f.used += rows > 0;
+        f.heavy += rows > 256;
         f.max_rows = rows > f.max_rows ? rows : f.max_rows;
         prev = gl[g];
     }
@@ -69,19 +72,21 @@ inline bool gmsq_skips_empty(const int64_t* gl, int64_t E, int64_t ntl, int64_t 
     return f.max_rows <= 192 || (f.mostly_empty() && f.tiles * ntl >= 2 * grid);
 }
 
-// The same question for the epilogue of the ring dequant GEMM (its SKIP instance): yes when every group
-// fits one tile, or when most fragments are empty.  Time with SKIP over without, 32 to 70000 rows:
-//   groups of at most 256 rows, valid share 0.25 to 0.9:   0.90 to 1.01
-//   groups past 256 rows, valid share under 0.56:          0.87 to 1.0
-//   groups past 256 rows, valid share 0.56 to 0.9:         0.97 to 1.09, by the length of K: 64 experts of
-//     2944 x 6464 with 336 rows on average 606 us without, 659 with; 256 experts of 1088 x 4672 with 273
-//     rows 857 against 902; 64 experts of 3328 x 6400 with 571 rows 956 against 924
+// The same question for the epilogue of the ring dequant GEMM (its SKIP instance): yes unless at least
+// half of the groups have more than one tile and 9 of 16 fragments are valid.  Time with SKIP over
+// without, 130 calls of 800 to 70000 rows:
+//   groups of at most 256 rows:                                     0.90 to 1.01
+//   under half of the groups past 256 rows (skewed routing):        0.87 to 1.01
+//   half of the groups or more past 256 rows, valid share under 0.56: 0.92 to 1.0
+//   the same, valid share 0.56 to 0.9:                              0.97 to 1.09: 64 experts of 2944 x 6464
+//     with 336 rows on average 606 us without, 659 with; 256 experts of 1088 x 4672 with 273 rows 857 against
+//     902; 64 experts of 3328 x 6400 with 571 rows 956 against 924
 // (a group's full and nearly empty tile again: with SKIP the light tiles' workgroups run ahead and
 // the row tiles of a group no longer meet at their weight slab).
 inline bool ring_skips_empty(const int64_t* gl, int64_t E)
 {
     const TileFill f = tile_fill(gl, E);
-    return f.max_rows <= 256 || f.mostly_empty();
+    return 2 * f.heavy < f.used || f.mostly_empty();
 }
 
 // Time model of a tiled GEMM for the rules that choose a tile: a tile alone on its CU takes p us per
@@ -100,15 +105,16 @@ inline double tile_rounds_us(int64_t tiles, double units, double p, double r, do
 // Estimated time in us of a BM x BN tile kernel over the call (tile_rounds_us: p us per 128 of K for a
 // tile alone on its CU, r in a full round of 256, o per tile); the bytes the call must move pass at
 // bw TB/s, partly hidden by the multiplications (the two times combine as the root of their
-// squares: powers of 3 and 4 fit worse); f us per call.  The
-// skinny kernel (at most 32 rows per group, in one or two blocks of 16), the 256 x 256 ring core (more
-// than 32 rows, batch 1, K of at least 256) and the 8-wave 256 x 256 kernel (more than 32 rows, other
-// batches and K) are candidates like the others.  Their constants are fits (bw and f need not be physical)
-// to 1700 shapes, 1 to 65536 rows, K 64 to 10240, N 64 to 16384, 1 to 256 groups, 1 to 32 batches, on
-// which every candidate was timed: the choice is 1.4% off the fastest on average.  Against taking no
-// tile at all one shape in a hundred loses more than 2% (1149 x 4672 x 14400, 129 against 117 us); with
-// the ring at 1.55 us per 128 of K and its constants for the 8-wave kernel too it was one in twenty,
-// up to 40% (1614 x 3648 x 12288, 111 against 95; 11288 x 208 x 1088, 19 against 14).  Measured:
+// squares: powers of 3 and 4 fit worse); f us per call.  The skinny kernel (at most 32 rows per group, in
+// one or two blocks of 16), the 256 x 256 ring core (more than 32 rows, batch 1, K of at least 256) and the
+// 8-wave 256 x 256 kernel (more than 32 rows, other batches and K) are candidates like the others.  The
+// constants are fits (bw and f need not be physical) to 1900 calls, 1 to 65536 rows, K 64 to 10240, N 64 to
+// 16384, 1 to 256 groups, evenly and unevenly filled, 1 to 32 batches, on which every candidate was timed:
+// the choice is 0.9% off the fastest on average.  Against taking no tile at all one call in a hundred loses
+// more than 2% (32 x (79 x 1728 x 832), 28 us against 24; 256 groups of 768 x 6656 with 1 row, at most 30,
+// 129 against 118); with the ring at 1.55 us per 128 of K and its constants for the 8-wave kernel too it was
+// one in sixteen, up to 40% (1614 x 3648 x 12288, 111 against 95; 11288 x 208 x 1088, 19 against 14).
+// Measured:
 //   us, by rows (dense 7168 x 4096)          us, by rows per expert (256 x 2048 x 7168, drawn unevenly)
 //                  24    300   1024  2048  4096       8     24    47    96    256
 //   32 x 64       19.2   39     96   189   379       803    -     -     -      -
@@ -131,11 +137,11 @@ struct DeqCand {
 };
 enum { DEQ_RING = 5, DEQ_SKINNY = 6, DEQ_LDS = 7, DEQ_SKINNY2 = 8 };  // 6, 8: one and two blocks of 16 rows
 inline constexpr DeqCand kDeqCand[] = {
-    {32, 64, 256, 0.30, 0.152, 1.5, 5.2, 2.0, 1.0},   {64, 128, 256, 0.36, 0.31, 2.7, 6.8, 2.0, 1.0},
-    {64, 256, 256, 0.63, 0.58, 4.9, 6.9, 1.85, 1.0},  {128, 128, 512, 0.34, 0.486, 6.8, 6.5, 2.0, 1.0},
-    {128, 256, 512, 0.55, 0.87, 10.6, 6.5, 2.0, 1.0}, {256, 256, 0, 1.21, 1.21, 12.0, 5.7, 3.0, 0.38},
-    {32, 256, 0, 0.85, 0.30, 1.0, 6.3, 3.0, 1.0},     {256, 256, 0, 1.33, 1.33, 4.4, 9.7, 3.7, 0.70},
-    {32, 256, 0, 1.00, 0.40, 2.0, 5.6, 3.0, 1.0},
+    {32, 64, 256, 0.30, 0.152, 1.5, 5.2, 2.0, 1.0},   {64, 128, 256, 0.30, 0.31, 2.7, 7.0, 2.9, 1.0},
+    {64, 256, 256, 0.66, 0.57, 4.2, 6.7, 1.2, 1.0},   {128, 128, 512, 0.34, 0.486, 6.8, 6.5, 2.0, 1.0},
+    {128, 256, 512, 0.31, 0.78, 8.9, 5.8, 1.62, 1.0}, {256, 256, 0, 1.07, 1.07, 12.9, 5.6, 3.7, 0.39},
+    {32, 256, 0, 0.85, 0.30, 1.0, 6.3, 3.0, 1.0},     {256, 256, 0, 0.92, 0.92, 5.7, 5.9, 5.3, 0.73},
+    {32, 256, 0, 0.70, 0.30, 6.0, 6.3, 3.0, 1.0},
 };
 
 // The index of the cheapest candidate, -1 where none fits a dispatch.

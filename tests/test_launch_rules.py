@@ -47,7 +47,7 @@ def test_dqsq_grid(rules, threads):
 # tile numbers of the rules: (rows, columns, threads)
 DEQ_TILES = [(32, 64, 256), (64, 128, 256), (64, 256, 256), (128, 128, 512), (128, 256, 512)]
 GMM_TILES = DEQ_TILES + [(256, 256, 512)]
-RING, SKINNY, LDS = 5, 6, 7  # the other kernels of the int8 rule
+RING, SKINNY, LDS, SKINNY2 = 5, 6, 7, 8  # the other kernels of the int8 rule
 
 
 def _one_group(M):
@@ -103,6 +103,7 @@ def test_gmsq_skip_rule(rules, counts, skips):
     ([33] * 64, True), ([129] * 16, True), ([256] * 8, True), ([224, 7, 0, 256], True),  # one tile per group
     ([274] * 256, False), ([336] * 64, False), ([571] * 64, False),  # a full and a lighter tile in each group
     ([600] + [40] * 31, True),                                       # mostly empty fragments
+    ([1000, 700, 400] + [224, 130, 90, 60] * 2, True),               # most groups of one tile
 ])
 def test_ring_skip_rule(rules, counts, skips):
     assert bool(rules.rule_ring_skips_empty(_gl(counts), len(counts))) is skips
@@ -115,6 +116,7 @@ def test_ring_skip_rule(rules, counts, skips):
     ([11288], 208, 1088, 1, LDS), ([1862], 96, 6976, 1, LDS), ([94], 832, 1280, 32, LDS), ([1362], 960, 1344, 4, LDS),
     # small products: tiles that fill the chip; few rows of many experts: the streaming kernel
     ([24], 7168, 4096, 1, 0), ([300], 7168, 4096, 1, 1), ([8] * 256, 2048, 7168, 1, SKINNY),
+    ([8] * 254 + [18, 2], 2048, 7168, 1, SKINNY2), ([29], 960, 1472, 32, 2),
 ])
 def test_dequant_kernel_choice(rules, counts, K, N, batch, kernel):
     assert rules.rule_pick_deq(_gl(counts), len(counts), sum(counts), K, N, batch, K >= 256) == kernel
