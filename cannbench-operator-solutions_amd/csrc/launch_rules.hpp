@@ -36,7 +36,6 @@ inline int64_t gmsq_decode_grid(int64_t groups, int64_t ntl, int64_t cus) { retu
 struct TileFill {
     int64_t frags = 0, tiles = 0, max_rows = 0;  // 32-row fragments with valid rows, 256-row tiles
     int64_t used = 0, heavy = 0;                 // groups with rows, with more than 256
-    bool mostly_empty() const { return 2 * frags < 9 * tiles; }  // under 9 of 16 fragments
 };
 
 inline TileFill tile_fill(const int64_t* gl, int64_t E)
@@ -57,19 +56,19 @@ inline TileFill tile_fill(const int64_t* gl, int64_t E)
 
 // Whether the GroupedMatmulSwigluQuant prefill kernel leaves out the publish and requant of 32-row
 // fragments without valid rows (its SKIP instance): yes when no 256-row tile is full enough to lose by it,
-// or when the empty fragments outweigh what full tiles lose and the tiles fill at least two rounds of
-// the grid (below that the call takes as long as its full tiles).  Measured gain of SKIP, by valid
+// or when most groups have one tile and enough fragments are empty.  Measured gain of SKIP, by valid
 // share of the fragments:
 //   256 x 7168 x 4096:  47 rows per expert (0.25) 1.035, 128 rows (0.5) 1.037, 192 (0.75) 1.016,
-//                       256 (1.0) 0.99, Zipf 128 on average (0.43) 1.025, Zipf 512 (0.81) level
+//                       256 (1.0) 0.99, Zipf 128 on average (0.43) 1.025, Zipf 512 (0.81) 1.004
 //   128 x 2048 x 2048:  47 rows 1.18, 128 rows 1.08, 300 rows (0.62) 0.93, 288 rows (0.56) 0.93
-//   64 x 2048 x 1536:   47 rows 1.22, 300 rows 0.95; 16 x 4096 x 2048, Zipf 64 (under two rounds) 0.97
+//   64 x 2048 x 1536:   47 rows 1.22, 300 rows 0.95; 64 x 1024 x 2048, 600 rows uneven (0.80) 1.06
+//   80 calls with Zipf routing (0.45 to 0.86, 70 to 5600 tiles): 0.99 to 1.09
 // Experts of just over 256 rows (a full tile and a nearly empty one, valid share 9/16 at least) lose
 // most: a workgroup meets the same kind of tile in every round, and the early ones run out of step.
-inline bool gmsq_skips_empty(const int64_t* gl, int64_t E, int64_t ntl, int64_t grid)
+inline bool gmsq_skips_empty(const int64_t* gl, int64_t E)
 {
     const TileFill f = tile_fill(gl, E);
-    return f.max_rows <= 192 || (f.mostly_empty() && f.tiles * ntl >= 2 * grid);
+    return f.max_rows <= 192 || (2 * f.heavy < f.used && 20 * f.frags < 17 * 8 * f.tiles);  // 0.85
 }
 
 // The same question for the epilogue of the ring dequant GEMM (its SKIP instance): yes unless at least
@@ -86,7 +85,7 @@ inline bool gmsq_skips_empty(const int64_t* gl, int64_t E, int64_t ntl, int64_t 
 inline bool ring_skips_empty(const int64_t* gl, int64_t E)
 {
     const TileFill f = tile_fill(gl, E);
-    return 2 * f.heavy < f.used || f.mostly_empty();
+    return 2 * f.heavy < f.used || 16 * f.frags < 9 * 8 * f.tiles;
 }
 
 // Time model of a tiled GEMM for the rules that choose a tile: a tile alone on its CU takes p us per

@@ -332,7 +332,7 @@ static int gmsq_impl(const int8_t* x, int64_t x_rows, const int32_t* row_index, 
         const int grid = (ntl == 16 && cus >= 256) ? 256 : (cus / ntl) * ntl;
         const bool gather = row_index != nullptr;
         const bool defer = (K + PfCfg::BK - 1) / PfCfg::BK >= kPfDeferMinStages;
-        const bool skip = gmsq_skips_empty(group_list, E, ntl, grid);
+        const bool skip = gmsq_skips_empty(group_list, E);
         const void* main_k = !defer   ? (gather ? (const void*)gmsq_prefill_kernel<true, false, false>
                                                 : (const void*)gmsq_prefill_kernel<false, false, false>)
                              : gather ? (skip ? (const void*)gmsq_prefill_kernel<true, true, true>

@@ -9,10 +9,7 @@ int rule_pick_deq(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N,
     return cb::pick_deq(gl, E, M, K, N, batch, ring_ok, 256);
 }
 int rule_pick_gmm(const int64_t* gl, int64_t E, int64_t M, int64_t K, int64_t N) { return cb::pick_gmm(gl, E, M, K, N, 256); }
-int rule_gmsq_skips_empty(const int64_t* gl, int64_t E, int64_t ntl, int64_t grid)
-{
-    return cb::gmsq_skips_empty(gl, E, ntl, grid);
-}
+int rule_gmsq_skips_empty(const int64_t* gl, int64_t E) { return cb::gmsq_skips_empty(gl, E); }
 int64_t rule_gmsq_decode_grid(int64_t groups, int64_t ntl, int64_t cus) { return cb::gmsq_decode_grid(groups, ntl, cus); }
 int rule_ring_skips_empty(const int64_t* gl, int64_t E) { return cb::ring_skips_empty(gl, E); }
 }

@@ -223,19 +223,20 @@ def test_int32_core_tile_bytes_past_4gib(cb):
 ])
 def test_prefill_instances_agree(cb, orc, counts, K, N, y_offset):
     """The prefill kernel has an instance that leaves out empty 32-row fragments and one that does not; the
-    call's groups choose.  A row's result depends on its own group alone: every group computed beside a group
-    of 256 full rows that makes the call take the other instance gives the same bits, and the call meets the
+    call's groups choose.  A row's result depends on its own group alone: every group computed beside two groups
+    of 300 rows that make the call take the other instance gives the same bits, and the call meets the
     oracle."""
     x, w, ws, xs, gl = _inputs(counts, K, N, sum(counts))
     y, ys, _ = _run_raw(cb, x, w, ws, xs, gl, y_offset)
     yr, ysr = orc.gmsq(x.cpu().numpy(), w.cpu().numpy(), ws.cpu().numpy(), xs.cpu().numpy(), np.array(gl))
     assert np.abs(y.cpu().numpy().astype(int) - yr).max() <= 1
     np.testing.assert_allclose(ys.cpu().numpy(), ysr, rtol=1e-5)
-    full = rand_i8((256, K), cpu_gen(1))
+    more = rand_i8((600, K), cpu_gen(1))
     for g in {0, 1, len(counts) - 1}:
         a, b = (gl[g - 1] if g else 0), gl[g]
         if b - a == 0:
             continue
-        yo, yso, _ = _run_raw(cb, torch.cat([x[a:b], full]), torch.stack([w[g], w[g]]), torch.stack([ws[g], ws[g]]),
-                              torch.cat([xs[a:b], xs.new_full((256,), 0.01)]), [b - a, b - a + 256], y_offset)
-        assert torch.equal(yo[:b - a], y[a:b]) and torch.equal(yso[:b - a], ys[a:b])
+        n = b - a
+        yo, yso, _ = _run_raw(cb, torch.cat([x[a:b], more]), torch.stack([w[g]] * 3), torch.stack([ws[g]] * 3),
+                              torch.cat([xs[a:b], xs.new_full((600,), 0.01)]), [n, n + 300, n + 600], y_offset)
+        assert torch.equal(yo[:n], y[a:b]) and torch.equal(yso[:n], ys[a:b])

@@ -25,7 +25,7 @@ def rules(tmp_path_factory):
     gl = ctypes.POINTER(i64)
     lib.rule_pick_deq.argtypes = [gl, i64, i64, i64, i64, i64, ctypes.c_int]
     lib.rule_pick_gmm.argtypes = [gl, i64, i64, i64, i64]
-    lib.rule_gmsq_skips_empty.argtypes = [gl, i64, i64, i64]
+    lib.rule_gmsq_skips_empty.argtypes = [gl, i64]
     lib.rule_ring_skips_empty.argtypes = [gl, i64]
     lib.rule_gmsq_decode_grid.argtypes = [i64, i64, i64]
     lib.rule_gmsq_decode_grid.restype = i64
@@ -89,14 +89,15 @@ def _gl(counts):
     ([33] * 64, True), ([47] * 256, True), ([192] * 8, True),          # no tile full enough to lose
     ([256] * 256, False), ([224] * 64, False), ([512] * 64, False),    # full tiles
     ([257] * 128, False), ([288] * 128, False), ([300] * 256, False),  # a full and a nearly empty tile each
-    ([300] + [40] * 255, True),                                        # many small groups beside a full tile
-    ([300] + [40] * 15, False),                                        # the same, under two rounds of the grid
+    ([300] + [40] * 255, True), ([300] + [40] * 15, True),             # small groups beside a full tile
+    ([1000, 700, 400] + [224, 130, 90, 60] * 2, True),                 # skewed: most groups of one tile
+    ([250] * 60 + [300] * 4, False),                                   # nearly full tiles
     ([0] * 200 + [0, 40, 0], True),
 ])
 def test_gmsq_skip_rule(rules, counts, skips):
     """Leaving out the empty fragments is taken where it gains (groups far below a tile) and not where it loses
     (full tiles; groups of just over a tile)."""
-    assert bool(rules.rule_gmsq_skips_empty(_gl(counts), len(counts), 16, 256)) is skips
+    assert bool(rules.rule_gmsq_skips_empty(_gl(counts), len(counts))) is skips
 
 
 @pytest.mark.parametrize("counts,skips", [
