@@ -283,8 +283,8 @@ __global__ __launch_bounds__(256, 1) void gpf_dequant_kernel(const GemmArgs a)
         v16i acc[4][4];  // defined by the K loop (its first MFMAs start from zero)
         const int nblk = (cur_t.vrows + 31) / 32;
         const int nv = __builtin_amdgcn_readfirstlane(nblk > wm ? min((nblk - wm + 1) / 2, 4) : 0);
-        // A later tile's loop starts with wait vmcnt(63): its first 28 DMAs were issued before the
-        // previous epilogue's 64 stores, so at most 63 outstanding operations means they landed.
+        // A later tile's loop starts without waiting for the previous epilogue's stores (8 to 32 per lane):
+        // its stage 0 landed before that epilogue began (pf_kloop).
         if (nv >= 4) pf_kloop<4, true, false>(cur, nxt, offs, nk, rb, smem, a_rd, b_rd, acc, wave, first);
         else if (nv == 3) pf_kloop<3, true, false>(cur, nxt, offs, nk, rb, smem, a_rd, b_rd, acc, wave, first);
         else if (nv == 2) pf_kloop<2, true, false>(cur, nxt, offs, nk, rb, smem, a_rd, b_rd, acc, wave, first);

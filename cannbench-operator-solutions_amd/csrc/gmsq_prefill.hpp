@@ -389,9 +389,12 @@ __device__ __forceinline__ void pf_kloop(const PfSrc& dma, const PfSrc& nxt, con
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    // stage 0 landed: the first tile of a workgroup waits for its DMAs; a later tile's prologue was
-    // drained by its predecessor's epilogue (every VMEM result waited for before its exchange), so
-    // only the barrier
+    // stage 0 landed: the first tile of a workgroup waits for its DMAs.  A later tile needs only the
+    // barrier: its stage 0 is stage nk of its predecessor, which half2(nk - 1) waited for and put
+    // behind a barrier.  Its other stages are waited for below, each half2(kt) leaving 2 * ISSUE operations
+    // outstanding, the number issued after stage kt + 1 when nothing but DMAs is issued; the counter falls
+    // in order of issue, so an epilogue's stores and loads among them, however many, make that wait
+    // longer, never too short.
     if (first) wait_vmcnt_barrier<2 * C::ISSUE + C::A_ISSUE>();
     else wait_vmcnt_barrier<63>();
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0) in the compiler's own accounting
@@ -620,8 +623,7 @@ __device__ __forceinline__ u32 pf_wait(const EpiArgs& e, u32* counter, const u32
 // loads and takes an agent-scope acquire fence once the count is complete (pf_wait).
 // A release written in the memory model instead (a release fence per wave and a release add)
 // compiles to `buffer_wbl2 sc1`, a write-back of the XCD's whole L2, five times per tile: measured
-// 4.06 -> 5.14 ms per prefill call.  The wait also drains the next tile's stage DMAs, which the
-// K loop's first wait relies on.
+// 4.06 -> 5.14 ms per prefill call.  The wait also drains the next tile's stage DMAs.
 __device__ __forceinline__ void pf_release_maxima() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 __device__ __forceinline__ void pf_arrive(u32* counter)

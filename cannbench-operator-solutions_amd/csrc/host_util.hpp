@@ -88,9 +88,10 @@ inline int check_launch()
 }
 
 // Test hooks (set by cb_set_test_overrides, per thread, until changed): a forced grid for the
-// persistent GEMM kernels (0: the CU count; < 0: persistent launch off), a poll limit for the
-// GroupedMatmulSwigluQuant exchange wait (0: the default), and the GEMM tile (1 to 5: a tile of
-// gemm_tile.hpp; 128: the 128 x 128 GroupedMatmul kernel; 0: automatic).
+// persistent GEMM kernels (0: the CU count; < 0: persistent launch off; any but 0 also keeps the dequant
+// GEMM from choosing a tile), a poll limit for the GroupedMatmulSwigluQuant exchange wait (0: the
+// default), and the GEMM tile (1 to 5: a tile of gemm_tile.hpp, for GroupedMatmul 6 too; 128: the
+// 128 x 128 GroupedMatmul kernel; 0 and what an operator does not have: automatic).
 struct TestOverrides {
     int persistent_grid = 0, exchange_spin_limit = 0, gmm_tile = 0;
 };

@@ -197,14 +197,15 @@ int cb_grouped_matmul_swiglu_quant_noalloc(const int8_t* x, const int8_t* weight
  *                        every workgroup walk many tiles); < 0 turns that
  *                        persistent launch off, and GroupedMatmulSwigluQuant then takes its
  *                        two-pass path (the one it takes when its fused grid cannot be resident).
+ *                        Any value but 0 also keeps the dequant GEMM from choosing a smaller tile.
  *   exchange_spin_limit  polls of the GroupedMatmulSwigluQuant row-maximum exchange before a tile
  *                        gives up and leaves its output to the fix-up launch (default 2^20, about
  *                        2 s); a small value exercises the fix-up path, a negative one makes every
  *                        wait give up at once (the fix-up launch then writes every tile).
  *   gmm_tile             1 to 6 force one tile of the tiled GEMM (32 x 64, 64 x 128, 64 x 256,
  *                        128 x 128, 128 x 256; 256 x 256 for GroupedMatmul only) where its shape
- *                        conditions hold; 128 forces the
- *                        128 x 128 register-staged GroupedMatmul kernel for every fp16/bf16 shape.
+ *                        conditions hold; 128 forces the 128 x 128 register-staged GroupedMatmul
+ *                        kernel for every fp16/bf16 shape.
  */
 void cb_set_test_overrides(int persistent_grid, int exchange_spin_limit, int gmm_tile);
 

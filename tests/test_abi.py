@@ -182,7 +182,7 @@ def test_launch_grid_limits(lib):
     assert so.cb_dynamic_quant(FAKE, 1, 1 << 23, 64, FAKE, FAKE, None) == L.CB_ERR_SHAPE
     assert so.cb_add_rms_norm_dynamic_quant(FAKE, FAKE, FAKE, 2, big, 64, 1e-6, FAKE, FAKE, FAKE, None) \
         == L.CB_ERR_SHAPE
-    # H = 6 is off the vector path (whose persistent grid is bounded): one block per row
+    # H = 6 is off the vector path (whose grid is bounded): one block per row
     assert so.cb_dequant_swiglu_quant(FAKE, 1, big, 12, None, None, None, 0, FAKE, FAKE, None) == L.CB_ERR_SHAPE
     assert so.cb_moe_gating_top_k_softmax(FAKE, 3, big, 8, None, 2, FAKE, FAKE, FAKE, None) == L.CB_ERR_SHAPE
 
