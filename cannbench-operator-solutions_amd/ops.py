@@ -20,6 +20,7 @@ Reference plugins mirrored (paths under operators/):
 """
 
 import array
+import functools
 
 import torch
 
@@ -59,12 +60,12 @@ def _raise_status(name, code):
         raise RuntimeError(f"{name}: {L.status_string(code)} (status {code})")
 
 
-def _empty(like, shape, dtype):
-    """An uninitialised plain tensor on like's device.  new_empty is the cheaper call, but on a subclass it
-    builds that subclass."""
+def _new(like):
+    """An allocator of uninitialised plain tensors on like's device, called as f(shape, dtype=...).  new_empty
+    is the cheaper call, but on a subclass it builds that subclass."""
     if type(like) is torch.Tensor:
-        return like.new_empty(shape, dtype=dtype)
-    return torch.empty(shape, dtype=dtype, device=like.device)
+        return like.new_empty
+    return functools.partial(torch.empty, device=like.device)
 
 
 _DTYPE_CODES = {torch.float16: L.CB_DT_FLOAT16, torch.bfloat16: L.CB_DT_BFLOAT16,
@@ -115,10 +116,8 @@ def add_rms_norm_dynamic_quant_meta(x1, x2, gamma, epsilon):
     _check(gamma.dim() == 1 and gamma.size(0) == x1.size(-1),
            "add_rms_norm_dynamic_quant: gamma must be 1-D with size == x1.size(-1).")
     _check(gamma.dtype == x1.dtype, "add_rms_norm_dynamic_quant: gamma dtype must match x1 dtype.")
-    y = _empty(x1, x1.shape, torch.int8)
-    x_out = torch.empty_like(x1)
-    scale = _empty(x1, x1.shape[:-1], torch.float32)
-    return y, x_out, scale
+    new = _new(x1)
+    return new(x1.shape, dtype=torch.int8), torch.empty_like(x1), new(x1.shape[:-1], dtype=torch.float32)
 
 
 def add_rms_norm_dynamic_quant(x1, x2, gamma, epsilon):
@@ -150,9 +149,8 @@ def dynamic_quant_meta(x):
     _check(x.dim() >= 2, "dynamic_quant requires a tensor with rank >= 2.")
     _check(x.dtype in (torch.float16, torch.bfloat16),
            "dynamic_quant only supports float16 / bfloat16 inputs.")
-    y = _empty(x, x.shape, torch.int8)
-    scale = _empty(x, x.shape[:-1], torch.float32)
-    return y, scale
+    new = _new(x)
+    return new(x.shape, dtype=torch.int8), new(x.shape[:-1], dtype=torch.float32)
 
 
 def dynamic_quant(x):
@@ -178,9 +176,8 @@ def grouped_matmul_swiglu_quant_meta(x, weight, weight_scale, x_scale, group_lis
     _check(weight.dim() == 3, "grouped_matmul_swiglu_quant: weight must be 3D [E, K, N]")
     M, N = x.size(0), weight.size(2)
     _check(N % 2 == 0, "grouped_matmul_swiglu_quant: N must be even")
-    y = _empty(x, (M, N // 2), torch.int8)
-    y_scale = _empty(x, (M,), torch.float32)
-    return y, y_scale
+    new = _new(x)
+    return new((M, N // 2), dtype=torch.int8), new((M,), dtype=torch.float32)
 
 
 def _validate_group_list(prefix, group_list, E, M, max_e):
@@ -215,8 +212,9 @@ def _gmsq(name, x, row_index, weight, weight_scale, x_scale, group_list):
     _check(weight.dim() == 3, f"{name}: weight must be 3D [E, K, N]")
     M = x.size(0) if row_index is None else row_index.numel()
     _check(weight.size(2) % 2 == 0, f"{name}: N must be even")
-    y = _empty(x, (M, weight.size(2) // 2), torch.int8)
-    y_scale = _empty(x, (M,), torch.float32)
+    new = _new(x)
+    y = new((M, weight.size(2) // 2), dtype=torch.int8)
+    y_scale = new((M,), dtype=torch.float32)
     K = x.size(1)
     E, N = weight.size(0), weight.size(2)
     if M == 0 or N == 0 or E == 0:
@@ -230,7 +228,7 @@ def _gmsq(name, x, row_index, weight, weight_scale, x_scale, group_list):
     _on_device(name, x, weight, weight_scale, x_scale, row_index)
     lib = L.load()
     ws_bytes = lib.cb_grouped_matmul_swiglu_quant_workspace_size(M, K, N, E)
-    ws = _empty(x, (ws_bytes,), torch.uint8)
+    ws = new((ws_bytes,), dtype=torch.uint8)
     gla, keep = _group_ptr(gl)
     if row_index is None:
         rc = lib.cb_grouped_matmul_swiglu_quant(
@@ -272,7 +270,7 @@ def quant_matmul_meta(x1, x2, scale, offset=None, pertoken_scale=None, bias=None
     _check(x1.size(-1) == x2.size(-2), "quant_matmul requires x1.size(-1) == x2.size(-2).")
     dt = torch.bfloat16 if output_dtype == "bfloat16" else torch.float16
     shape = list(x1.shape[:-1]) + [x2.size(-1)]
-    return _empty(x1, shape, dt)
+    return _new(x1)(shape, dtype=dt)
 
 
 def quant_matmul(x1, x2, scale, *, offset=None, pertoken_scale=None, bias=None, output_dtype=None):
@@ -363,7 +361,7 @@ def grouped_matmul_meta(x, weight, group_list, bias=None, split_item=0, transpos
     N = weight.size(1) if transpose_weight else weight.size(2)
     _check(len(group_list) == E, "grouped_matmul: group_list length must equal the number of experts")
     ends = _gmm_ends(group_list, E, M)
-    y = _empty(x, (M, N), x.dtype)
+    y = _new(x)((M, N), dtype=x.dtype)
     return _gmm_outputs(y, ends, split_item)
 
 
@@ -390,7 +388,7 @@ def grouped_matmul(x, weight, group_list, bias=None, split_item=0, transpose_wei
         _check(bias.numel() == E * N, f"{name}: bias must have shape [E, N]")
     _check(x.dtype in _GMM_DTYPES and weight.dtype == x.dtype, f"{name}: unsupported dtype")
     _check(bias is None or bias.dtype in _GMM_DTYPES, f"{name}: unsupported dtype")
-    y = _empty(x, (M, N), x.dtype)
+    y = _new(x)((M, N), dtype=x.dtype)
     out = _gmm_outputs(y, ends, split_item)
     if M == 0 or N == 0:
         return out
@@ -409,7 +407,7 @@ def grouped_matmul(x, weight, group_list, bias=None, split_item=0, transpose_wei
 def grouped_matmul_quant_meta(x, weight, weight_scale, x_scale, group_list):
     _check(x.dim() == 2, "grouped_matmul: x must be 2D [M, K]")
     _check(weight.dim() == 3, "grouped_matmul: weight must be 3D [E, K, N] or [E, N, K]")
-    return _empty(x, (x.size(0), weight.size(2)), torch.bfloat16)
+    return _new(x)((x.size(0), weight.size(2)), dtype=torch.bfloat16)
 
 
 def grouped_matmul_quant(x, weight, weight_scale, x_scale, group_list):
@@ -470,7 +468,7 @@ def grouped_matmul_int32(x, weight, group_list):
     E, N = weight.size(0), weight.size(2)
     _check(weight.size(1) == K, f"{name}: K mismatch between x and weight")
     gl = _validate_group_list(name, group_list, E, M, L.CB_MAX_EXPERTS)
-    c = _empty(x, (M, N), torch.int32)
+    c = _new(x)((M, N), dtype=torch.int32)
     if M == 0 or N == 0:
         return c
     _on_device(name, x, weight)
@@ -489,10 +487,11 @@ def moe_re_routing_meta(tokens, expert_token_num_per_rank, per_token_scales=None
     _check(expert_token_num_per_rank.dim() == 2, "moe_re_routing: expert_token_num_per_rank must be 2D (N, E).")
     a, h = tokens.shape
     e = expert_token_num_per_rank.size(1)
-    return (_empty(tokens, (a, h), tokens.dtype),
-            _empty(tokens, (a,), torch.float32),
-            _empty(tokens, (a,), torch.int32),
-            _empty(expert_token_num_per_rank, (e,), expert_token_num_per_rank.dtype))
+    new = _new(tokens)
+    return (new((a, h), dtype=tokens.dtype),
+            new((a,), dtype=torch.float32),
+            new((a,), dtype=torch.int32),
+            _new(expert_token_num_per_rank)((e,), dtype=expert_token_num_per_rank.dtype))
 
 
 def moe_re_routing(tokens, expert_token_num_per_rank, per_token_scales=None, expert_token_num_type=1, idx_type=0):
@@ -547,7 +546,7 @@ def _mfr_resolve(epr, esdr, scales):
 def moe_finalize_routing_meta(expanded_permuted_rows, expanded_src_to_dst_row, skip1=None, skip2=None, bias=None,
                               scales=None, expert_for_source_row=None, drop_pad_mode=0):
     num_rows, _, H = _mfr_resolve(expanded_permuted_rows, expanded_src_to_dst_row, scales)
-    return _empty(expanded_permuted_rows, (num_rows, H), expanded_permuted_rows.dtype)
+    return _new(expanded_permuted_rows)((num_rows, H), dtype=expanded_permuted_rows.dtype)
 
 
 _FLOATS = (torch.float16, torch.float32, torch.bfloat16)
@@ -562,7 +561,7 @@ def moe_finalize_routing(expanded_permuted_rows, expanded_src_to_dst_row, skip1=
     epr = expanded_permuted_rows.contiguous()
     esdr = expanded_src_to_dst_row.contiguous()
     num_rows, K, H = _mfr_resolve(epr, esdr, scales)
-    out = _empty(epr, (num_rows, H), epr.dtype)
+    out = _new(epr)((num_rows, H), dtype=epr.dtype)
     if num_rows <= 0 or H <= 0 or K <= 0:
         return out
     num_dst = epr.numel() // H
@@ -602,8 +601,8 @@ def dequant_swiglu_quant_meta(x, weight_scale=None, activation_scale=None, quant
     _check(x.dim() == 2, "dequant_swiglu_quant requires a 2D input [TokensNum, 2H].")
     M, N2 = x.shape
     _check(N2 % 2 == 0, "dequant_swiglu_quant requires an even last dimension.")
-    return (_empty(x, (M, N2 // 2), torch.int8),
-            _empty(x, (M,), torch.float32))
+    new = _new(x)
+    return new((M, N2 // 2), dtype=torch.int8), new((M,), dtype=torch.float32)
 
 
 def dequant_swiglu_quant(x, weight_scale=None, activation_scale=None, quant_scale=None, activate_left=False):
@@ -657,9 +656,8 @@ def moe_gating_top_k_softmax_meta(x, finished=None, k=1):
     if finished is not None:
         _check(finished.dtype == torch.bool, f"{_MGT} requires a bool 'finished' tensor.")
     shape = tuple(x.shape[:-1]) + (k,)
-    return (_empty(x, shape, x.dtype),
-            _empty(x, shape, torch.int32),
-            _empty(x, shape, torch.int32))
+    new = _new(x)
+    return new(shape, dtype=x.dtype), new(shape, dtype=torch.int32), new(shape, dtype=torch.int32)
 
 
 def moe_gating_top_k_softmax(x, finished=None, k=1):
